@@ -442,11 +442,9 @@ def measure_prefill(args, backend, T, torch, workload, cpu_budget):
         roof = {"bound": "hbm", "achieved": round(byts / kern_us / 1e3, 1),
                 "peak": HBM_PEAK_GBS, "unit": "GB/s"}
     roof["frac"] = round(roof["achieved"] / roof["peak"], 4)
-    # past 64 rows (TBH_PREFILL_F16_MIN) the f16 forms: runtime-layout INT4
-    # on the weight-side kernel, fp32 x as two f16 pieces
-    f16 = M >= int(os.environ.get("TBH_PREFILL_F16_MIN") or 65) and (
-        prec == "int4kn" or (f32 and os.environ.get("TBH_PREFILL_F32_PIECES") != "4"))
-    kern = "gemm_ngw" if prec == "int4kn" and f16 else "gemm_bf16"
+    # past 64 rows the f16 forms: runtime-layout INT4, fp32 x as two f16 pieces
+    f16 = M > 64 and (prec == "int4kn" or f32)
+    kern = "gemm_bf16" if M <= 64 and (f32 or prec == "int4kn") else "gemm"
     x_form = ("fp32 x, two f16 pieces" if f16 else "fp32 x, three bf16 pieces") if f32 else "bf16 x"
     roof.update({"traffic": profiled_traffic(prec, N, K, M, "prefill_f32" if f32 else "prefill"),
                  "kernel": f"{kern} {N}x{K} M={M} ({pool[0].path}, {x_form})",

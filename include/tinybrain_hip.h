@@ -211,9 +211,9 @@ tbh_status tbh_weight_get_info(const tbh_weight *w, tbh_weight_info *info);
  * outputs (16, 32 or a multiple of 64 rows, or one block) run on the bf16
  * MFMA GEMM with every fp32 x row split exactly into three bf16 pieces (for
  * the runtime layout, x times the N-block's per-k scale, one fp32 rounding,
- * then split); past 64 rows INT8 rows and INT4 K-groups take x as two f16
- * pieces, scaled by a power of two per row, holding it to 2^-22 of the row's
- * largest element, on the f16 MFMA.  The GEMV kernels stage a row of
+ * then split); past 64 rows x is taken as two f16 pieces, scaled by a power
+ * of two per row, holding it to 2^-22 of the row's largest element, on the
+ * f16 MFMA.  The GEMV kernels stage a row of
  * x in LDS, so a K past about 13 K (INT8) or 14.5 K (INT4) elements runs on
  * the MFMA GEMM at every M (runtime-layout INT4 of such a K keeps the
  * reference's flat array and runs on the generic kernel); a long K that is
@@ -225,8 +225,8 @@ tbh_status tbh_matmul(tbh_device *dev, const float *x, int64_t M, int64_t K,
 /* Same product on device pointers, enqueued on `stream` (a hipStream_t of the
  * weight's device; NULL = the null stream).  Returns after the launch.
  * Launches that split K (matrix-core GEMV, MFMA GEMM) keep their partial sums,
- * and the MFMA GEMM past 64 rows its per-row exponents of x (an int32 per
- * row), in a workspace the library allocates per (device, stream) on first use and
+ * and the MFMA GEMM its 16-bit pieces of fp32 x (4 or 6 bytes per element, up
+ * to 128 MiB at a time) and their exponents (an int32 per row), in a workspace the library allocates per (device, stream) on first use and
  * keeps, with every buffer it outgrew, until tbh_device_close (a graph
  * captured on the stream may still hold them): a caller that creates many
  * short-lived streams should reuse a few, or call
@@ -278,8 +278,8 @@ tbh_status tbh_linear_device(const tbh_weight *w, const float *x, int64_t M,
  * exactly into three bf16 pieces), accumulation is fp32.  INT4 runtime
  * layout past 64 rows runs on f16 MFMA: the dequantized weight fl(q * s),
  * scaled by a power of two per N-block, as two f16 pieces holding it to
- * 2^-21 of itself, against x scaled by a power of two per row (exact), with
- * a pass over x for the row exponents in the stream's workspace.  x is [M, K] row-major bf16 bits
+ * 2^-21 of itself, against x scaled by a power of two per row (exact), a pass
+ * that writes x so, 2 bytes per element, to the stream's workspace.  x is [M, K] row-major bf16 bits
  * (16-byte aligned, K % 8 == 0), y is [M, N] fp32, both device pointers;
  * enqueued on `stream`.  TBH_E_UNSUPPORTED for weights outside the INT8
  * row / INT4 K-group / INT4 runtime-layout paths (tbh_weight_info.path), for

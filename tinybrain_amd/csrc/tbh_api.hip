@@ -19,8 +19,7 @@
 // address, looked up once per device in tbh_device_open) until the process
 // ends.  Host code only ever uses that looked-up address: the array's name
 // in host code is a host-side stand-in, not device memory.
-static constexpr size_t kNoAllocScratchBytes = size_t(16) << 20;
-static __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
+static __device__ __align__(256) unsigned char scratch[tbh::kNoAllocScratchBytes];
 
 namespace tbh {
 
@@ -425,7 +424,7 @@ hipError_t upload(T **dst, const T *src, size_t count, int64_t &bytes, int64_t &
 void free_weight(tbh_weight *w) {
     if (!w) return;
     for (void *p : {(void *)w->data, (void *)w->scales, (void *)w->zp, (void *)w->raw, (void *)w->raw_scales,
-                    (void *)w->raw_zp, (void *)w->ng_sexp})
+                    (void *)w->raw_zp, (void *)w->ng_sexp, (void *)w->ng_scaled})
         (void)hipFree(p);
     delete w;
 }
@@ -593,13 +592,20 @@ tbh_status tbh_weight_create(tbh_device *dev, const tbh_qtensor_desc *desc, tbh_
                     int e2 = 0;
                     if (mx > 0.0f) (void)std::frexp(mx, &e2);
                     ex[(size_t)nb] = e2;
-                    const float lo_ok = std::ldexp(1.0f, e2 - 36);
-                    for (int64_t k = 0; k < K && !w->ng_wide; ++k) {
-                        const float a = std::fabs(t[nb * w->Kp + k]);
-                        w->ng_wide = a > 0.0f && a < lo_ok;
-                    }
                 }
                 if (e == hipSuccess) e = upload(&w->ng_sexp, ex.data(), ex.size(), w->device_bytes, w->n_ng_sexp);
+                // The scales as the prefill GEMM stages them, times 2^(8 - e):
+                // exact, but for scales more than 2^36 under their block's
+                // bound, which are kept at 2^-28 so that no nonzero weight
+                // leaves the f16 range.
+                for (int64_t nb = 0; nb < NB; ++nb)
+                    for (int64_t k = 0; k < K; ++k) {
+                        float &v = t[nb * w->Kp + k];
+                        if (v == 0.0f || !std::isfinite(v)) continue;
+                        v = std::copysign(std::max(std::ldexp(std::fabs(v), 8 - ex[(size_t)nb]), 0x1p-28f), v);
+                    }
+                int64_t n_scaled = 0;
+                if (e == hipSuccess) e = upload(&w->ng_scaled, t.data(), t.size(), w->device_bytes, n_scaled);
                 w->stream_bytes = (count + 1) / 2 + 4 * d.n_scales;
             }
         } else {
@@ -805,32 +811,44 @@ static int64_t sgemv_min_rows(const tbh_weight &w) {
     return 9;
 }
 
-// Fewest rows of fp32 x that go to the MFMA GEMM (each row split exactly into
-// three bf16 pieces; launch_prefill_f32) instead of the GEMV kernels, which
-// stream the whole weight once per 2..8 rows.  Measured crossovers, us per
-// call GEMV / GEMM: INT8 5632x2048 M = 8 13.5 / 10.9; INT8 2048x2048 M = 8
-// 7.5 / 7.9, M = 12 10.7 / 8.0; INT4 2048x2048 M = 12 11.4 / 10.1 (M = 8
-// 7.8 / 9.7); INT4 4096x11008 M = 32 61.0 / 44.6; INT4 11008x4096 M = 32
-// 56.5 / 49.9 (M = 24 42.2 / 49.1); INT4 32000x2048 M = 64 101.7 / 67.5
-// (M = 48 76.5 / 78.4).
-// Runtime-layout INT4 has no matrix-core GEMV, so its GEMV route is the VALU
-// kernel four rows per launch: GEMM from 8 rows (2048x5632 M = 8 21.9 /
-// 13.8, 11008x4096 42.4 / 38.5) or 12 on weights under 8 Mi elements and on
-// N >= 16384 (2048x2048 M = 8 8.5 / 9.3, M = 12 12.5 / 9.4; 32000x2048 M = 8
-// 35.0 / 40.0, M = 12 49.6 / 39.2).
-//
+// Fewest rows of fp32 x that go to the MFMA GEMM (launch_prefill_f32) instead
+// of the GEMV kernels, which stream the whole weight once per 1..8 rows.
+// Measured crossovers, us per call GEMV / GEMM:
+//   INT4 (its matrix-core GEMV takes eight rows a launch): 2048x2048 16 rows
+//     11.8 / 12.8, 20 14.8 / 11.8 (12 is kept: 11.9 / 12.0 there);
+//     11008x4096 9 rows 21.5 / 24.1, 12 26.9 / 24.2; 4096x11008 12 rows 25.3 /
+//     24.7; 32000x2048 16 rows 26.0 / 30.7, 20 36.9 / 31.9, but 20000x1024 12
+//     rows 22.3 / 18.1; 32000x4096 9 rows 45.5 / 48.4, 12 54.7 / 49.0.
+//   INT8: 2048x2048 8 rows 7.5 / 7.9, 12 10.7 / 8.0; 4096x4096 4 rows 11.7 /
+//     12.3, 6 13.9 / 12.4; 2048x5632 4 rows 11.6 / 13.1, 6 15.3 / 12.1;
+//     5632x2048 8 rows 9.2 / 11.2 (one eight-row launch), 9 12.5 / 11.7;
+//     11008x4096 4 rows 22.3 / 20.5; 4096x11008 4 rows 48.1 / 22.0; 32000x2048
+//     4 rows 17.1 / 27.6, 6 31.6 / 25.0; 20000x1024 6 rows 11.8 / 13.6;
+//     32000x4096 4 rows 58.1 / 38.1.
+//   Runtime layout (four or eight rows a launch on the VALU): 2048x2048 9
+//     rows 11.5 / 11.5; 2048x5632 4 rows 11.4 / 13.2, 6 15.5 / 13.4; 4096x4096
+//     4 rows 15.2 / 14.3; 4096x11008 4 rows 34.1 / 27.6; 11008x4096 6 rows 29.8
+//     / 38.0, 8 42.5 / 38; 32000x2048 9 rows 39.6 / 42.5, 12 49.7 / 43.0;
+//     32000x4096 4 rows 53.9 / 72, 6 77.0 / 70.
 // burst8: the weight takes eight rows of this x in one burst GEMV launch
-// (gemv8_supported).  Below 16384 outputs that launch beats the GEMM at
-// exactly 8 rows (us per call, GEMM / one 8-row launch: INT8 5632x2048 11.2
-// / 9.2, 11264x2048 15.4 / 15.7; runtime-layout INT4 5632x2048 13.1 / 9.9;
-// INT8 32000x2048 27.4 / 32.4), so those weights start the GEMM at 9.
+// (gemv8_supported), which beats the GEMM at up to eight rows below 16384
+// outputs.
 static int64_t mfma_min_rows(const tbh_weight &w, bool burst8) {
-    const int64_t nk = w.N * w.K;
-    const bool big = nk >= ((int64_t)8 << 20);
-    if (w.path == Path::Int4NGroup) return big && w.N < 16384 ? (burst8 ? 9 : 8) : 12;
-    if (w.precision == TBH_PREC_INT8) return big ? (burst8 && w.N < 16384 ? 9 : 8) : 12;
-    if (nk <= ((int64_t)24 << 20)) return 12;
-    return w.N >= 16384 ? 64 : 32;
+    const int64_t nk = w.N * w.K, mi = (int64_t)1 << 20;
+    const bool wide = w.N >= 16384;
+    if (w.path == Path::Int4NGroup) {
+        if (nk < 8 * mi) return 12;
+        if (wide) return nk >= 100 * mi ? 6 : 12;
+        if (burst8) return 9;
+        return w.K >= 8192 ? 4 : nk >= 32 * mi ? 8 : 6;
+    }
+    if (w.precision == TBH_PREC_INT8) {
+        if (nk < 8 * mi) return 12;
+        if (wide) return nk >= 100 * mi ? 4 : nk >= 32 * mi ? 6 : 8;
+        if (burst8) return 9;
+        return nk >= 32 * mi ? 4 : 6;
+    }
+    return wide && nk > 24 * mi && nk < 100 * mi ? 17 : 12;
 }
 
 static tbh_status matmul_enqueue(const tbh_weight *w, const float *x, int64_t M, float *y,

@@ -112,10 +112,9 @@ struct tbh_weight {
     // scales (0 when all are zero), for the prefill GEMM's f16 scaling
     int32_t *ng_sexp = nullptr;
     int64_t n_ng_sexp = 0;
-    // some N-block holds a nonzero finite scale below 2^(e - 36), so that a
-    // weight 16 q s 2^(8 - e) can fall under the f16 range: the prefill GEMM
-    // takes a variant that floors such scales (gemm_ngw with FLOOR)
-    bool ng_wide = false;
+    // Int4NGroup: the scale table times 2^(8 - ng_sexp), nonzero entries at
+    // least 2^-28 in magnitude, as the prefill GEMM stages it
+    float *ng_scaled = nullptr;
     bool mfma_tiles = false;     // data in 1 KiB MFMA tiles (else K-contiguous rows)
 
     // generic path: the reference arrays as given
@@ -194,6 +193,9 @@ struct FusedGemvArgs {
 bool gemv_fused_supported(const tbh_weight &w);
 hipError_t launch_gemv_fused(const tbh_weight &w, const FusedGemvArgs &f, hipStream_t s);
 
+// Scratch of the no-allocation entry.
+constexpr size_t kNoAllocScratchBytes = size_t(16) << 20;
+
 // MFMA dequant-GEMV for 2 <= M <= 8 rows of x on row-layout INT4 K-group
 // weights without zero points (tbh_sgemv.hip).  launch_sgemv returns
 // hipErrorInvalidValue for shapes it does not take (odd alignment of x,
@@ -217,13 +219,21 @@ hipError_t launch_prefill(const tbh_weight &w, const uint16_t *x, int64_t ldx, i
                           int64_t ldy, hipStream_t s, const Scratch &scr);
 
 // The same GEMM for fp32 x [M][ldx] (16-byte aligned rows, K % 8 == 0):
-// each x row is split exactly into three bf16 pieces and a zero
-// row, the four rows go through the bf16 MFMAs, and the epilogue adds each
-// row's four results; past 64 rows of INT8-row or INT4 K-group weights, two
-// f16 pieces of x scaled per row on the f16 MFMA (tbh_prefill.hip).
+// each x row is split exactly into three bf16 pieces (a few rows of a small
+// weight: staged with a zero row by the bf16 GEMM itself); past 64 rows, two
+// f16 pieces of x scaled per row on the f16 MFMA (tbh_gemm.hip).
 // hipErrorInvalidValue for weights or shapes it does not take.
 hipError_t launch_prefill_f32(const tbh_weight &w, const float *x, int64_t ldx, int64_t M, float *y,
                               int64_t ldy, hipStream_t s, const Scratch &scr);
+
+// The step-DMA prefill GEMM (tbh_gemm.hip): fp32 x as two f16 pieces per row,
+// bf16 x as given (runtime-layout INT4: one f16 piece); M rows whose pieces
+// (gemm_pieces_bytes) fit scr, else hipErrorNotReady before any launch.
+bool gemm_supported(const tbh_weight &w);
+size_t gemm_pieces_bytes(const tbh_weight &w, bool f32, int64_t rows);
+hipError_t launch_gemm(const tbh_weight &w, const void *x, bool f32, int64_t ldx, int64_t M, float *y, int64_t ldy,
+                       hipStream_t s, const Scratch &scr);
+hipError_t launch_split_sum(const float *part, int splits, float *y, int64_t n, int64_t cus, hipStream_t s);
 
 // Device workspace of at least `bytes` owned by (dev, stream), grown on
 // demand (tbh_api.hip).  Growing allocates a new buffer and keeps the old one
