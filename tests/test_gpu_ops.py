@@ -147,6 +147,56 @@ def test_attention(backend, case):
     np.testing.assert_allclose(y, R.attention(q, k, v, None, hd, nh, nkv), rtol=1e-4, atol=1e-5)
 
 
+# (batch, seq, kv, head_dim, heads, kv_heads): the matrix-core kernel takes 64
+# (query, query head) rows per block in groups of 16, and tiles of 32 positions
+# (64 at head_dim 32) halved between two waves; it needs 96 Ki (224 Ki at
+# head_dim 64) of (query, quad of heads, position)
+TILE_CASES = [
+    (2, 1600, 32, 32, 1, 1),         # the fewest positions: only the first wave of each group has any
+    (2, 65, 897, 64, 2, 2),          # one row past a block; ranges over blocks, one position over
+    (2, 63, 512, 32, 3, 3),          # one row short of a block
+    (1, 1025, 113, 64, 4, 2),        # a last tile of one position past the first wave's half
+    (1, 80, 321, 128, 4, 4),         # rows end on a group of 16
+    (2, 33, 1000, 64, 16, 2),        # eight query heads per key/value head, ranges merged
+    (1, 50, 1000, 128, 24, 2),       # twelve query heads per key/value head, ranges
+    (1, 300, 513, 32, 12, 12),
+    (1, 16, 6144, 128, 1, 1),        # the fewest rows: three groups of 16 empty
+    (1, 16, 6143, 128, 1, 1),        # just below the line: the one-wave-per-row kernel
+]
+
+
+@pytest.mark.parametrize("case", TILE_CASES)
+@pytest.mark.parametrize("masked", [False, True])
+def test_attention_tiles(backend, case, masked):
+    B, S, Tk, hd, nh, nkv = case
+    q, k, v = (_rand(S + Tk + i, (B, n, h * hd)) for i, n, h in ((0, S, nh), (1, Tk, nkv), (2, Tk, nkv)))
+    mask = None
+    if masked:
+        mask = _rand(5, (Tk,))
+        mask[:Tk // 2] = -np.inf                          # whole leading tiles without a position
+        mask[Tk // 2::7] = np.finfo(np.float32).min       # weight 0, but a finite score
+        mask[-1] = 0.5
+    y = backend.attention(q, k, v, mask, hd, nh, nkv)
+    # scores and sums in fp32: hd products of size ~1 shift a score by at most
+    # hd^1/2 * 2^-24 * |s| ~ 4e-6, the weights and output by the same share
+    np.testing.assert_allclose(y, R.attention(q, k, v, mask, hd, nh, nkv), rtol=1e-4, atol=1e-5)
+
+
+def test_attention_tiles_special_values(backend):
+    S, Tk, hd, nh = 1500, 84, 64, 2
+    q, k, v = _rand(1, (S, nh * hd)), _rand(2, (Tk, nh * hd)), _rand(3, (Tk, nh * hd))
+    assert np.all(np.isnan(backend.attention(q, k, v, np.full(Tk, -np.inf, np.float32), hd, nh, nh)))
+    low = np.full(Tk, np.finfo(np.float32).min, np.float32)   # swallows the scores: the mean of v
+    np.testing.assert_allclose(backend.attention(q, k, v, low, hd, nh, nh),
+                               np.tile(v.mean(0, dtype=np.float64), (S, 1)), rtol=1e-4, atol=1e-5)
+    v[-1, 5] = np.inf                                     # the last position: not repeated past the end
+    y = backend.attention(q, k, v, None, hd, nh, nh)
+    assert np.all(y[:, 5] == np.inf) and np.all(np.isfinite(np.delete(y, 5, 1)))
+    q[3, :hd] = np.nan                                    # one row of one head
+    y = backend.attention(q, k, v, None, hd, nh, nh)
+    assert np.all(np.isnan(y[3, :hd])) and not np.any(np.isnan(np.delete(y, 3, 0)))
+
+
 def test_attention_masks(backend):
     S, Tk, hd, nh, nkv = 16, 16, 16, 4, 4
     q, k, v = _rand(1, (S, nh * hd)), _rand(2, (Tk, nkv * hd)), _rand(3, (Tk, nkv * hd))

@@ -14,7 +14,9 @@
 // Attention: when there are too few (query, key/value head) pairs to fill
 // the chip, the key positions are split over several blocks, each writing a
 // partial (max, sum, output) per head to a workspace, and a second kernel
-// merges them (split-KV decoding).  Head dimensions 16/32/64/128 take one
+// merges them (split-KV decoding).  Many query rows at head dimension
+// 32/64/128 go to the matrix cores in tiles (attention_tile, by the rule at
+// use_tiles).  Otherwise head dimensions 16/32/64/128 take one
 // wave per (query, query head, range): the four waves of a block are query
 // heads of one key/value head and share its rows through L1.  Other head
 // dimensions that are multiples of 4 take a block per (query, key/value
@@ -738,6 +740,310 @@ __global__ __launch_bounds__(256) void attention_wave(const GrpArgs g) {
     }
 }
 
+// Attention of many query rows for head_dim HD in {32, 64, 128}, on the fp32
+// matrix instruction (v_mfma_f32_16x16x4_f32: operands, products and sums are
+// the fp32 the one-wave-per-row kernel uses; only the order of the sums
+// differs).  Bound by that instruction, 256 flop per clock and CU (2.1 GFLOP
+// of a 512-token prompt, 32 heads of 64: 14 us), and by the softmax between
+// the two products, which runs on the same waves.  us per call, attention_wave /
+// this (batch, queries, positions, heads, key/value heads, head_dim):
+//   1 512 512 32 4 64    161 / 40     1 512 512 32 32 128     1180 / 67
+//   1 100 700 32 4 64     59 / 21.6   2 1000 1500 32 32 128  13947 / 633
+//   1 64 512 12 12 64   16.9 / 15.4   1 16 1000 32 8 128        37 / 30
+//   1 512 512 8 2 32      22 / 12.7   2 1000 1500 8 2 32       203 / 59
+//
+// A (query, query head) pair of a key/value head is a row; a block takes 64
+// rows and one range of positions.  Eight waves: four groups of 16 rows, each
+// twice, the two waves of a group taking the halves of every POS-position
+// tile and merging at the end.  Tiles of keys and values are read once per
+// block (attention_wave reads them once per row) and staged in two LDS
+// buffers, the next tile's global loads outstanding while this one is
+// multiplied, one barrier a tile.
+//
+// Operands need no shuffle.  Scores are formed transposed, keys x q: lane
+// (g = lane / 16, n = lane % 16) then holds positions 4g + i of query row n,
+// which is the layout the second product wants for its right operand when its
+// i-th instruction takes positions {i, 4 + i, 8 + i, 12 + i}.  Max, sum and
+// rescale factor belong to one row n per lane; the max takes two exchanges.
+// The head dimension is dealt so that all LDS reads are 16 bytes (8 at HD 32):
+// keys, piece 4g of every 16; values, VW consecutive ones per lane, so the
+// lane ends with 4 VW consecutive outputs.  Sums are short chains joined by a
+// tree (8 products, 8 positions, then the tile, then the running sum): the
+// error against float64 is 1.4e-7 to 2.0e-7, attention_wave's 1.6e-7 to 4.3e-7
+// on the same calls; single chains gave 2.5e-7 to 5e-7 and the same time.
+// Tiles of 64 positions at HD 64 spill; two blocks per CU by splitting the
+// positions of 256 tiles in two gain nothing over the merge (41.7 us for 40.3).
+// LDS rows are padded by 4 floats:
+// 16 rows at one column then cover all 64 banks.
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+struct TileArgs {
+    GrpArgs g;
+    int64_t nrows;     // seq_len * rep: rows of one (batch, key/value head)
+    int64_t rtiles;    // ceil(nrows / 64): blocks per head and range
+    int64_t heads;     // batch * nkv
+    int64_t sums;      // floats of (max, sum) pairs before the p.v sums in the partials
+};
+
+template <int HD>
+__global__ __launch_bounds__(512, HD == 128 ? 2 : 4) void attention_tile(const TileArgs ta) {
+    constexpr int PT = HD >= 64 ? 1 : 2;           // 16-position pieces per wave and tile
+    constexpr int POS = 32 * PT;                    // positions per tile
+    constexpr int LD = HD + 4;                      // floats per LDS row
+    constexpr int VW = HD >= 64 ? 4 : HD / 16, NH = HD / 16 / VW;
+    constexpr int NLD = POS * HD / 4 / 512;         // 16-byte loads per thread for keys, as many for values
+    __shared__ __attribute__((aligned(16))) float lds[2][2][POS * LD];
+    const GrpArgs &g = ta.g;
+    const AttnArgs &a = g.a;
+    const int tid = threadIdx.x, w = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+    const int gg = lane >> 4, n = lane & 15;
+    const int rg = w & 3, ks = w >> 2;
+    // the heads run fastest, so that one head's blocks meet in few L2s
+    int64_t bi = blockIdx.x;
+    const int64_t bh = bi % ta.heads;
+    bi /= ta.heads;
+    const int split = (int)(bi % g.splits);
+    const int64_t row0 = bi / g.splits * 64 + rg * 16;
+    const int64_t batch = bh / a.nkv;
+    const int kvh = (int)(bh % a.nkv);
+    const int64_t kvd = (int64_t)a.nkv * HD;
+    const float *kb = a.k + batch * a.kv_len * kvd + (int64_t)kvh * HD;
+    const float *vb = a.v + batch * a.kv_len * kvd + (int64_t)kvh * HD;
+    const int64_t c0 = split * g.chunk, c1 = min(a.kv_len, c0 + g.chunk);
+    const bool live = row0 < ta.nrows;              // uniform over the wave
+    const int64_t row = min(row0 + n, ta.nrows - 1);
+    const int64_t bq = batch * a.seq_len + row / g.rep;
+    const int hg = (int)(row % g.rep);
+    const int head = kvh * g.rep + hg;
+
+    float q[HD / 4];                                // q rows need not be 16-byte aligned
+    {
+        const float *qrow = a.q + (bq * a.nh + head) * HD + 4 * gg;
+#pragma unroll
+        for (int j = 0; j < HD / 16; ++j)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) q[4 * j + c] = qrow[16 * j + c];
+    }
+    f32x4 kr[NLD], vr[NLD];
+    int64_t off[NLD];
+#pragma unroll
+    for (int j = 0; j < NLD; ++j) {
+        const int e = tid + 512 * j;
+        off[j] = e / (HD / 4) * kvd + 4 * (e % (HD / 4));
+    }
+    auto fetch = [&](int64_t p0) {
+        const float *kp = kb + p0 * kvd, *vp = vb + p0 * kvd;      // uniform
+        if (p0 + POS <= c1) {
+#pragma unroll
+            for (int j = 0; j < NLD; ++j) {
+                kr[j] = *(const f32x4 *)(kp + off[j]);
+                vr[j] = *(const f32x4 *)(vp + off[j]);
+            }
+        } else {
+            const int left = (int)(c1 - p0);
+#pragma unroll
+            for (int j = 0; j < NLD; ++j) {
+                const int e = tid + 512 * j, r = e / (HD / 4), c = e % (HD / 4);
+                const int64_t o1 = min(r, left - 1) * kvd + 4 * c;
+                kr[j] = *(const f32x4 *)(kp + o1);
+                vr[j] = *(const f32x4 *)(vp + o1);
+                if (r >= left) vr[j] = f32x4{0.f, 0.f, 0.f, 0.f};   // their weight is 0: keep 0 * inf out
+            }
+        }
+    };
+    auto stage = [&](int b) {
+#pragma unroll
+        for (int j = 0; j < NLD; ++j) {
+            const int e = tid + 512 * j, r = e / (HD / 4), c = e % (HD / 4);
+            *(f32x4 *)&lds[b][0][r * LD + 4 * c] = kr[j];
+            *(f32x4 *)&lds[b][1][r * LD + 4 * c] = vr[j];
+        }
+    };
+
+    float m = -INFINITY, l = 0.0f;                  // l: this lane's positions only
+    f32x4 o[NH * VW];
+#pragma unroll
+    for (int i = 0; i < NH * VW; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+    fetch(c0);
+    stage(0);
+    __syncthreads();
+    int buf = 0;
+    for (int64_t p0 = c0; p0 < c1; p0 += POS, buf ^= 1) {
+        const bool more = p0 + POS < c1;
+        if (more) fetch(p0 + POS);
+        const int64_t w0 = p0 + ks * 16 * PT;       // this wave's first position
+        if (live && w0 < c1) {
+            const float *kt = &lds[buf][0][ks * 16 * PT * LD], *vt = &lds[buf][1][ks * 16 * PT * LD];
+            f32x4 mk[PT], s[PT][HD / 16];
+            if (a.mask)
+#pragma unroll
+                for (int t = 0; t < PT; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) mk[t][i] = a.mask[min(w0 + 16 * t + 4 * gg + i, c1 - 1)];
+#pragma unroll
+            for (int j = 0; j < HD / 16; ++j)
+#pragma unroll
+                for (int t = 0; t < PT; ++t) {
+                    const f32x4 kk = *(const f32x4 *)&kt[(16 * t + n) * LD + 16 * j + 4 * gg];
+                    f32x4 s0 = f32x4{0.f, 0.f, 0.f, 0.f}, s1 = s0;   // sums of 8 products, then a tree
+                    s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[0], q[4 * j], s0, 0, 0, 0);
+                    s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[2], q[4 * j + 2], s1, 0, 0, 0);
+                    s0 = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[1], q[4 * j + 1], s0, 0, 0, 0);
+                    s1 = __builtin_amdgcn_mfma_f32_16x16x4f32(kk[3], q[4 * j + 3], s1, 0, 0, 0);
+                    s[t][j] = s0 + s1;
+                }
+#pragma unroll
+            for (int d = 1; d < HD / 16; d *= 2)
+#pragma unroll
+                for (int t = 0; t < PT; ++t)
+#pragma unroll
+                    for (int j = 0; j < HD / 16; j += 2 * d) s[t][j] += s[t][j + d];
+#pragma unroll
+            for (int t = 0; t < PT; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    s[t][0][i] *= a.scale;
+                    if (a.mask) s[t][0][i] += mk[t][i];
+                }
+            if (w0 + 16 * PT > c1) {
+                const int left = (int)(c1 - w0);
+#pragma unroll
+                for (int t = 0; t < PT; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        if (16 * t + 4 * gg + i >= left) s[t][0][i] = -INFINITY;
+            }
+            float nm = m;
+#pragma unroll
+            for (int t = 0; t < PT; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) nm = fmaxf(nm, s[t][0][i]);
+            nm = fmaxf(nm, __shfl_xor(nm, 16));
+            nm = fmaxf(nm, __shfl_xor(nm, 32));
+            if (__any(nm != -INFINITY)) {           // else every position so far is masked
+                const float ref = nm == -INFINITY ? 0.0f : nm;
+                const float corr = expf(m - ref);
+                m = nm;
+                l *= corr;
+#pragma unroll
+                for (int t = 0; t < PT; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        s[t][0][i] = expf(s[t][0][i] - ref);
+                        l += s[t][0][i];
+                    }
+                // sums of eight positions, added up before they join the running one
+                f32x4 pv[2 * PT][NH * VW];
+#pragma unroll
+                for (int t = 0; t < PT; ++t)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int h = 0; h < NH; ++h) {
+                            const float *vp = &vt[(16 * t + 4 * gg + i) * LD + 64 * h + VW * n];
+                            float vv[VW];
+                            __builtin_memcpy(vv, __builtin_assume_aligned(vp, 4 * VW), sizeof vv);
+#pragma unroll
+                            for (int c = 0; c < VW; ++c) {
+                                f32x4 &d = pv[2 * t + i / 2][h * VW + c];
+                                d = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                    vv[c], s[t][0][i], i % 2 ? d : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                            }
+                        }
+#pragma unroll
+                for (int x = 0; x < NH * VW; ++x) {
+                    f32x4 sum = pv[0][x] + pv[1][x];
+                    if constexpr (PT == 2) sum += pv[2][x] + pv[3][x];
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) o[x][i] = o[x][i] * corr + sum[i];
+                }
+            }
+        }
+        if (more) stage(buf ^ 1);
+        __syncthreads();
+    }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+
+    // the second wave of each row group hands its part to the first
+    constexpr int XR = NH * VW * 4 + 2;
+    static_assert(4 * XR * 64 <= 4 * POS * LD, "parts fit the tile buffers");
+    float *xb = &lds[0][0][0] + rg * XR * 64 + lane;
+    if (ks == 1) {
+        xb[0] = m;
+        xb[64] = l;
+#pragma unroll
+        for (int x = 0; x < NH * VW; ++x)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) xb[64 * (2 + 4 * x + i)] = o[x][i];
+    }
+    __syncthreads();
+    if (ks == 1 || row0 + n >= ta.nrows) return;
+    const float m1 = xb[0], mm = fmaxf(m, m1);
+    const float e0 = m == -INFINITY ? 0.0f : expf(m - mm), e1 = m1 == -INFINITY ? 0.0f : expf(m1 - mm);
+    l = l * e0 + xb[64] * e1;
+#pragma unroll
+    for (int x = 0; x < NH * VW; ++x)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) o[x][i] = o[x][i] * e0 + xb[64 * (2 + 4 * x + i)] * e1;
+
+    // lane (gg, n): outputs 64 h + 4 VW gg + (VW i + c) of row n
+    float *dst;
+    if (g.splits == 1) {
+        const float den = l + kAttnEps;
+        const bool dead = mm == -INFINITY;          // kv_len > 0 here: all masked gives NaN
+#pragma unroll
+        for (int x = 0; x < NH * VW; ++x)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) o[x][i] = dead ? NAN : o[x][i] / den;
+        dst = a.out + (bq * a.nh + head) * HD;
+    } else {
+        const int64_t slot = (bq * a.nh + head) * g.splits + split;
+        if (gg == 0) *(float2 *)&g.part[2 * slot] = float2{mm, l};
+        dst = g.part + ta.sums + slot * HD;
+    }
+#pragma unroll
+    for (int h = 0; h < NH; ++h)
+#pragma unroll
+        for (int b = 0; b < VW; ++b) {
+            f32x4 r;
+#pragma unroll
+            for (int d = 0; d < 4; ++d) r[d] = o[h * VW + (4 * b + d) % VW][(4 * b + d) / VW];
+            *(f32x4 *)(dst + 64 * h + 4 * VW * gg + 4 * b) = r;
+        }
+}
+
+// Merges attention_tile's partials, [row][split] of (max, sum) and of p.v sums,
+// as attention_combine does: HD / 4 threads per output row, so a block takes
+// 1024 / HD rows (attention_combine takes a block per row and eight head slots
+// per key/value head, 7 of them empty with as many key/value as query heads).
+template <int HD>
+__global__ __launch_bounds__(256) void attention_tile_merge(const TileArgs ta) {
+    const GrpArgs &g = ta.g;
+    const int64_t row = (int64_t)blockIdx.x * (1024 / HD) + threadIdx.x / (HD / 4);
+    const int d4 = threadIdx.x % (HD / 4);
+    if (row >= g.a.rows) return;
+    const float2 *ml = (const float2 *)g.part + row * g.splits;
+    const f32x4 *ov = (const f32x4 *)(g.part + ta.sums + row * g.splits * HD) + d4;
+    float mm = -INFINITY, l = 0.0f;
+    for (int sp = 0; sp < g.splits; ++sp) mm = fmaxf(mm, ml[sp].x);
+    f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+    for (int sp = 0; sp < g.splits; ++sp) {
+        const float2 p = ml[sp];
+        const float e = p.x == -INFINITY ? 0.0f : expf(p.x - mm);
+        const f32x4 v = ov[sp * (HD / 4)];
+        l += e * p.y;
+        o += e * v;
+    }
+    const float den = l + kAttnEps;
+    f32x4 r;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) r[i] = mm == -INFINITY ? NAN : o[i] / den;
+    *((f32x4 *)(g.a.out + row * HD) + d4) = r;
+}
+
 // Merges the split partials of attention_group / attention_wave: per head,
 // M = max m_s, out = sum(o_s e^(m_s - M)) / (sum(l_s e^(m_s - M)) + eps).
 // One block per (unit, head); thread (sg, d4) loads the partials of splits
@@ -885,6 +1191,49 @@ hipError_t launch_act(const tbh_device *dev, const float *x, int64_t n, float *y
 
 hipError_t launch_attention_rows(const AttnArgs &a, hipStream_t s);
 
+// Whether a call's rows go to attention_tile: at least one full group of 16 per
+// key/value head (so no single query of up to 15 heads per key/value head,
+// where a group's matrix work is mostly padding), and enough (block, position)
+// pairs of attention_wave that its reads of every key and value row for each
+// of them outweigh the tile kernel's start and merge.  us, attention_wave /
+// attention_tile, below and above the line: HD 64, 16 x 1000 positions of 32
+// heads on 4 (125 Ki) 17.6 / 20.0, of 12 on 12 (188 Ki) 17.1 / 18.8, 64 x 512
+// of 32 on 4 (256 Ki) 24.9 / 16.5; HD 32, 64 x 512 of 8 on 2 (64 Ki) 10.2 /
+// 11.0, 100 x 700 (137 Ki) 15.1 / 13.2; HD 128, 64 x 64 of 32 on 8 (32 Ki)
+// 11.6 / 12.8, 16 x 1000 (125 Ki) 36.8 / 28.5.
+bool use_tiles(const TileArgs &ta, int64_t wave_blocks) {
+    const GrpArgs &g = ta.g;
+    return ta.nrows >= 16 && g.a.kv_len >= 32 &&
+           wave_blocks * g.a.kv_len >= (g.a.hd == 64 ? 224 : 96) * 1024;
+}
+
+template <int HD>
+hipError_t launch_attention_tile(tbh_device *dev, TileArgs &ta, hipStream_t s) {
+    GrpArgs &g = ta.g;
+    const AttnArgs &a = g.a;
+    const int64_t tiles = ta.rtiles * ta.heads, cus = std::max(1, dev->cu_count);
+    // one block per CU (eight waves), each with at least 128 positions
+    const int64_t want = std::min<int64_t>(std::min(cus / tiles, a.kv_len / 128), 64);
+    if (want > 1) {
+        g.chunk = ((a.kv_len + want - 1) / want + 63) / 64 * 64;
+        g.splits = (int32_t)((a.kv_len + g.chunk - 1) / g.chunk);
+        ta.sums = (2 * a.rows * g.splits + 3) / 4 * 4;
+        const size_t bytes = (size_t)(ta.sums + a.rows * g.splits * HD) * sizeof(float);
+        if (g.splits > 1) g.part = (float *)stream_workspace(dev, s, bytes);
+        if (!g.part) {   // no workspace (graph capture before any eager call): one split
+            g.splits = 1;
+            g.chunk = a.kv_len;
+        }
+    }
+    if (tiles * g.splits > INT32_MAX) return hipErrorInvalidValue;
+    hipLaunchKernelGGL(attention_tile<HD>, dim3((unsigned)(tiles * g.splits)), dim3(512), 0, s, ta);
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess || g.splits == 1) return e;
+    constexpr int R = 1024 / HD;
+    hipLaunchKernelGGL(attention_tile_merge<HD>, dim3((unsigned)((a.rows + R - 1) / R)), dim3(256), 0, s, ta);
+    return hipGetLastError();
+}
+
 hipError_t launch_attention(tbh_device *dev, const AttnArgs &a, hipStream_t s) {
     if (a.hd % 4 != 0 || !aligned16(a.k) || !aligned16(a.v) || !aligned16(a.out)) return launch_attention_rows(a, s);
     GrpArgs g{};
@@ -898,6 +1247,20 @@ hipError_t launch_attention(tbh_device *dev, const AttnArgs &a, hipStream_t s) {
     // blocks per split: (query row, KV head, 4 query heads) for attention_wave,
     // (query row, KV head, 8 query heads) for attention_group
     const int64_t per_split = wave ? (a.rows / a.nh) * a.nkv * ((g.rep + 3) / 4) : g.units;
+    if (a.kv_len > 0 && (a.hd == 32 || a.hd == 64 || a.hd == 128)) {
+        TileArgs ta{};
+        ta.nrows = a.seq_len * g.rep;
+        ta.rtiles = (ta.nrows + 63) / 64;
+        ta.heads = a.rows / a.nh / std::max<int64_t>(a.seq_len, 1) * a.nkv;
+        ta.g = g;
+        if (use_tiles(ta, per_split)) {
+            switch (a.hd) {
+            case 32: return launch_attention_tile<32>(dev, ta, s);
+            case 64: return launch_attention_tile<64>(dev, ta, s);
+            default: return launch_attention_tile<128>(dev, ta, s);
+            }
+        }
+    }
     const int64_t target = 2 * (int64_t)std::max(1, dev->cu_count);
     if (per_split < target && a.kv_len > 64) {
         const int64_t want =
