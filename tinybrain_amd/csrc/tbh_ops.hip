@@ -770,7 +770,8 @@ __global__ __launch_bounds__(256) void attention_wave(const GrpArgs g) {
 // lane ends with 4 VW consecutive outputs.  Sums are short chains joined by a
 // tree (8 products, 8 positions, then the tile, then the running sum): the
 // error against float64 is 1.4e-7 to 2.0e-7, attention_wave's 1.6e-7 to 4.3e-7
-// on the same calls; single chains gave 2.5e-7 to 5e-7 and the same time.
+// on the same calls; single chains gave 1.4e-7 to 5.5e-7 for 35 and 62 us
+// in place of 40 and 67.
 // Tiles of 64 positions at HD 64 spill; two blocks per CU by splitting the
 // positions of 256 tiles in two gain nothing over the merge (41.7 us for 40.3).
 // LDS rows are padded by 4 floats:
