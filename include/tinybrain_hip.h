@@ -226,7 +226,8 @@ tbh_status tbh_matmul(tbh_device *dev, const float *x, int64_t M, int64_t K,
  * weight's device; NULL = the null stream).  Returns after the launch.
  * Launches that split K (matrix-core GEMV, MFMA GEMM) keep their partial sums,
  * and the MFMA GEMM its 16-bit pieces of fp32 x (4 or 6 bytes per element, up
- * to 128 MiB at a time) and their exponents (an int32 per row), in a workspace the library allocates per (device, stream) on first use and
+ * to 128 MiB at a time: longer x is taken in even parts) and their exponents
+ * (an int32 per row), in a workspace the library allocates per (device, stream) on first use and
  * keeps, with every buffer it outgrew, until tbh_device_close (a graph
  * captured on the stream may still hold them): a caller that creates many
  * short-lived streams should reuse a few, or call

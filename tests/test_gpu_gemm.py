@@ -13,6 +13,7 @@ import numpy as np
 import pytest
 
 import oracle as O
+from launches import gemms, launches
 from tinybrain_amd import _abi
 import tinybrain_amd as T
 from test_gpu_sweep import _oracle_weight, _weight
@@ -118,3 +119,38 @@ def test_small_scratch_same_bits(backend, kind, K, N, M):
             backend.set_option(_abi.OPT_NOALLOC_SCRATCH_BYTES, 0)
         assert torch.equal(y.view(torch.int32), ref.view(torch.int32)), (kind, K, N, M, limit)
     _check(ref.cpu().numpy(), x.cpu().numpy(), _oracle_weight(qt, pq.layout), (kind, K, N, M))
+
+
+# fp32 x of long prompts, whose pieces pass 128 MiB and are made in parts: 4096
+# rows at K = 8192, 3008 at K = 11008
+@pytest.mark.parametrize("kind,K,M", [
+    ("int4_kn_g32", 8192, 4033),
+    ("int4_kn_g32", 8192, 4096),
+    ("int4_kn_g32", 8192, 4097),
+    ("int4_kn_g32", 11008, 3072),
+    ("int8", 8192, 4160),
+    ("int4_nk_g32", 8192, 4033),
+    ("int4_nk_g32", 8192, 4100),
+])
+def test_pieces_in_parts(backend, kind, K, M):
+    import torch
+
+    N = 64
+    qt, pq = _weight(kind, K, N, seed=K + M)
+    w = backend.weight(pq)
+    x = torch.from_numpy(O.fill_normal(29 * K + M, M * K).reshape(M, K)).cuda()
+    y, stream = torch.empty((M, N), device="cuda"), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    backend.matmul_device(x, w, out=y, stream=stream)
+    torch.cuda.synchronize()
+    ls = launches(lambda: backend.matmul_device(x, w, out=y, stream=stream), stream)
+    # every part on the GEMM, in one form, with at most the pieces before it and
+    # a sum after it
+    assert {n for n, _, _ in ls} <= {"x_pieces", "gemm", "split_sum", "tail_sum"}, ls
+    assert {g.pieces for g in gemms(ls)} == {2}, ls
+    most = (128 << 20) // (64 * 4 * (-(-K // 64) * 64)) * 64
+    assert len(gemms(ls)) == -(-M // most) and len(ls) <= 3 * len(gemms(ls)), ls
+    _check(y.cpu().numpy(), x.cpu().numpy(), _oracle_weight(qt, pq.layout), (kind, K, N, M))
+    z = backend.matmul_device_noalloc(x, w, out=torch.empty_like(y))
+    torch.cuda.synchronize()
+    assert torch.equal(z.view(torch.int32), y.view(torch.int32))

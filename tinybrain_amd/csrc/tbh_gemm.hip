@@ -154,11 +154,6 @@ hipError_t launch_split_x(const void *x, bool f32, int xp, int64_t ldx, int32_t 
                : launch_pieces<false>(x, ldx, K, rows, e, out, ldp, piece_stride, s);
 }
 
-// Product pieces per x row: bf16 x one; fp32 x two f16 pieces (22 bits of x)
-// past 64 rows, three bf16 pieces (all of it, as the GEMV kernels read x) up
-// to 64, where the third costs little: the weights' bytes are the bound.
-int x_count(bool f32, int64_t M) { return !f32 ? 1 : M > 64 ? 2 : 3; }
-
 // The tail's sums: element e of tail tile r (four at a time) = tail_part[0]
 // [r][e] + tail_part[1][r][e] + ..., in part order, written where the tile
 // lies inside the output.
@@ -284,13 +279,24 @@ bool gemm_supported(const tbh_weight &w) {
            w.n_scales_dev * (int64_t)sizeof(float) < (int64_t)kDead;
 }
 
-// Bytes of scratch that `rows` rows of x take as pieces (with their row
-// exponents ahead of them): none for bf16 x on INT8 rows and INT4 K-groups.
-size_t gemm_pieces_bytes(const tbh_weight &w, bool f32, int64_t rows) {
-    if (!f32 && w.path != Path::Int4NGroup) return 0;
+// 16-bit pieces per x row that a product of M rows writes to scratch: none of
+// bf16 x on INT8 rows and INT4 K-groups (read as given), one of bf16 x on
+// runtime-layout INT4; fp32 x two f16 pieces (22 bits of x) past 64 rows, three
+// bf16 pieces (all of it, as the GEMV kernels read x) up to 64, where the third
+// costs little: the weights' bytes are the bound.  M is the whole product's:
+// its parts (gemm_rows) are all of one form.
+int gemm_pieces(const tbh_weight &w, bool f32, int64_t M) {
+    if (!f32) return w.path == Path::Int4NGroup ? 1 : 0;
+    return M > 64 ? 2 : 3;
+}
+
+// Bytes of scratch that `rows` rows of x take as pieces, with their row
+// exponents ahead of them.
+size_t gemm_pieces_bytes(const tbh_weight &w, int pieces, int64_t rows) {
+    if (pieces == 0) return 0;
     const int64_t ldp = (w.K + kBK - 1) / kBK * kBK;
     const size_t eb = ((size_t)rows * sizeof(int32_t) + 255) / 256 * 256;
-    return eb + ((size_t)(x_count(f32, rows) * rows * ldp) * 2 + 255) / 256 * 256;
+    return eb + ((size_t)(pieces * rows * ldp) * 2 + 255) / 256 * 256;
 }
 
 static hipError_t launch_kind(const Args &a, int kind, int xp, const Plan &pl, int64_t blocks, hipStream_t s) {
@@ -355,11 +361,13 @@ static hipError_t launch_seq(Args a, int kind, int xp, const Plan &pl, const voi
 }
 
 // hipErrorNotReady, before anything is enqueued, when the pieces' scratch is
-// not to be had.
-hipError_t launch_gemm(const tbh_weight &w, const void *x, bool f32, int64_t ldx, int64_t M, float *y, int64_t ldy,
-                       hipStream_t s, const Scratch &scr) {
+// not to be had; hipErrorInvalidConfiguration, likewise, for pieces that no
+// tile of the weight's kind takes (three on runtime-layout INT4, which
+// prefill's rule never asks for).
+hipError_t launch_gemm(const tbh_weight &w, const void *x, bool f32, int nx, int64_t ldx, int64_t M, float *y,
+                       int64_t ldy, hipStream_t s, const Scratch &scr) {
     const int kind = w.path == Path::Int8Row ? W8 : w.path == Path::Int4KGroup ? W4K : W4N;
-    const int xp = x_count(f32, M);
+    const int xp = std::max(nx, 1);
     const int64_t cus = std::max(1, w.dev->cu_count);
     Args a{};
     a.y = y;
@@ -384,7 +392,8 @@ hipError_t launch_gemm(const tbh_weight &w, const void *x, bool f32, int64_t ldx
 
     // scratch: the pieces of x, then the partial tiles
     Plan pl = choose(kind, xp, M, w.N, a.nsteps, cus, ldy == w.N);
-    const size_t pieces = gemm_pieces_bytes(w, f32, M);
+    if (pl.sps == 0) return hipErrorInvalidConfiguration;
+    const size_t pieces = gemm_pieces_bytes(w, nx, M);
     const int64_t n = M * w.N;
     size_t part_bytes = pl.splits > 1 ? (size_t)(pl.splits * n) * sizeof(float)
                                       : (size_t)pl.tail_parts * pl.tail_r * (16 * pl.tm) * (128 * pl.tn) * sizeof(float);

@@ -226,13 +226,15 @@ hipError_t launch_prefill(const tbh_weight &w, const uint16_t *x, int64_t ldx, i
 hipError_t launch_prefill_f32(const tbh_weight &w, const float *x, int64_t ldx, int64_t M, float *y,
                               int64_t ldy, hipStream_t s, const Scratch &scr);
 
-// The step-DMA prefill GEMM (tbh_gemm.hip): fp32 x as two f16 pieces per row,
-// bf16 x as given (runtime-layout INT4: one f16 piece); M rows whose pieces
-// (gemm_pieces_bytes) fit scr, else hipErrorNotReady before any launch.
+// The step-DMA prefill GEMM (tbh_gemm.hip) on M rows of x, taken as `pieces`
+// 16-bit pieces per row (gemm_pieces of the whole product; 0: bf16 x as given),
+// whose scratch (gemm_pieces_bytes) scr has to hold, else hipErrorNotReady
+// before any launch.
 bool gemm_supported(const tbh_weight &w);
-size_t gemm_pieces_bytes(const tbh_weight &w, bool f32, int64_t rows);
-hipError_t launch_gemm(const tbh_weight &w, const void *x, bool f32, int64_t ldx, int64_t M, float *y, int64_t ldy,
-                       hipStream_t s, const Scratch &scr);
+int gemm_pieces(const tbh_weight &w, bool f32, int64_t M);
+size_t gemm_pieces_bytes(const tbh_weight &w, int pieces, int64_t rows);
+hipError_t launch_gemm(const tbh_weight &w, const void *x, bool f32, int pieces, int64_t ldx, int64_t M, float *y,
+                       int64_t ldy, hipStream_t s, const Scratch &scr);
 hipError_t launch_split_sum(const float *part, int splits, float *y, int64_t n, int64_t cus, hipStream_t s);
 
 // Device workspace of at least `bytes` owned by (dev, stream), grown on

@@ -837,24 +837,25 @@ static bool keep_gemm_bf16(const tbh_weight &w, int64_t rows) {
            (8 * tiles == cus || 4 * tiles == cus);
 }
 
-// Rows of x per launch_gemm call whose pieces need scratch: kPiecesBytes of
-// them, and 64 at least.
-constexpr size_t kPiecesBytes = (size_t)128 << 20;
-static int64_t gemm_rows_per_call(const tbh_weight &w, bool f32) {
-    const size_t per64 = gemm_pieces_bytes(w, f32, 128) / 2;
-    if (per64 == 0) return kGemmRowsPerLaunch;
-    return std::min<int64_t>(kGemmRowsPerLaunch, std::max<int64_t>(1, (int64_t)(kPiecesBytes / per64)) * 64);
-}
-
-// x [M][ldx] (fp32, or bf16) through launch_gemm in calls of `rows` rows;
+// x [M][ldx] (fp32, or bf16) through launch_gemm, in calls whose pieces take
+// kPiecesBytes at most (or 64 rows).  The calls share the rows evenly: a short
+// last one would run a small product's plan behind a large one's.
 // hipErrorNotReady, with nothing enqueued, when scratch is not to be had.
+constexpr size_t kPiecesBytes = (size_t)128 << 20;
 static hipError_t gemm_rows(const tbh_weight &w, const void *x, bool f32, int64_t ldx, int64_t M, float *y, int64_t ldy,
                             hipStream_t s, const Scratch &scr) {
-    const int64_t rows = gemm_rows_per_call(w, f32);
+    const int pieces = gemm_pieces(w, f32, M);
+    int64_t most = kGemmRowsPerLaunch;
+    if (pieces > 0) {
+        const int64_t per64 = (int64_t)(64 * pieces * 2) * ((w.K + 63) / 64 * 64);
+        most = std::min(most, std::max<int64_t>(1, (int64_t)kPiecesBytes / per64) * 64);
+    }
+    const int64_t calls = (M + most - 1) / most;
+    const int64_t rows = ((M + calls - 1) / calls + 63) / 64 * 64;
     for (int64_t m0 = 0; m0 < M; m0 += rows) {
         const int64_t mc = std::min(rows, M - m0);
-        const hipError_t e = launch_gemm(w, (const char *)x + m0 * ldx * (f32 ? 4 : 2), f32, ldx, mc, y + m0 * ldy, ldy,
-                                         s, scr);
+        const hipError_t e = launch_gemm(w, (const char *)x + m0 * ldx * (f32 ? 4 : 2), f32, pieces, ldx, mc,
+                                         y + m0 * ldy, ldy, s, scr);
         if (e != hipSuccess) return m0 > 0 && e == hipErrorNotReady ? hipErrorOutOfMemory : e;
     }
     return hipSuccess;
@@ -870,7 +871,7 @@ hipError_t launch_prefill_f32(const tbh_weight &w, const float *x, int64_t ldx, 
     // capture before any eager call).
     // (16 rows of pieces fit the no-allocation entry's scratch, so that its
     // results are the device entry's)
-    if (gemm_supported(w) && use_gemm(w, M) && gemm_pieces_bytes(w, true, 16) <= kNoAllocScratchBytes) {
+    if (gemm_supported(w) && use_gemm(w, M) && gemm_pieces_bytes(w, 3, 16) <= kNoAllocScratchBytes) {
         const hipError_t e = gemm_rows(w, x, true, ldx, M, y, ldy, s, scr);
         if (e != hipErrorNotReady) return e;
     }
