@@ -12,6 +12,7 @@ import numpy as np
 import pytest
 
 import tinybrain_amd as T
+from launches import launches
 from oracle import ops_ref as R
 from tinybrain_amd import _abi
 from tinybrain_amd.quantized import PreconditionFailure
@@ -195,6 +196,73 @@ def test_attention_tiles_special_values(backend):
     q[3, :hd] = np.nan                                    # one row of one head
     y = backend.attention(q, k, v, None, hd, nh, nh)
     assert np.all(np.isnan(y[3, :hd])) and not np.any(np.isnan(np.delete(y, 3, 0)))
+
+
+def _attention_kernel(backend, case, aligned=True):
+    """The first kernel that an attention call of this shape launches."""
+    import torch
+
+    B, S, Tk, hd, nh, nkv = case
+    q, k, v, out = (torch.zeros(n, device="cuda") for n in (B * S * nh * hd, B * Tk * nkv * hd,
+                                                           B * Tk * nkv * hd + 1, B * S * nh * hd))
+    sh, s = _abi.AttentionShape(B, S, Tk, hd, nh, nkv), torch.cuda.Stream()
+    ptr = [q.data_ptr(), k.data_ptr(), v.data_ptr() + (0 if aligned else 4)]
+    torch.cuda.synchronize()
+
+    def call():
+        assert backend._lib.tbh_attention_device(backend._dev, ctypes.byref(sh), *ptr, None, out.data_ptr(),
+                                                 ctypes.c_void_p(s.cuda_stream)) == _abi.OK
+    call()                                                # its workspace
+    torch.cuda.synchronize()
+    return launches(call, s)[0].name
+
+
+# one shape per head dimension on the matrix-core kernel, by the rule at use_tiles
+TILE_HD = [(1, 1500, 300, 32, 4, 4), (1, 600, 300, 64, 8, 2), (1, 100, 1300, 128, 4, 2)]
+
+
+@pytest.mark.parametrize("case", TILE_HD)
+def test_attention_tiles_nan_scores(backend, case):
+    """A NaN score is no masked one: positions whose keys or mask are NaN give NaN,
+    also where a whole tile of them comes first."""
+    assert _attention_kernel(backend, case) == "attention_tile"
+    B, S, Tk, hd, nh, nkv = case
+    q, k, v = (_rand(40 + i, (B, n, h * hd)) for i, n, h in ((0, S, nh), (1, Tk, nkv), (2, Tk, nkv)))
+    for lo, hi in ((0, 16), (0, 32), (0, 64), (16, 32), (Tk - 1, Tk)):
+        kn = k.copy()
+        kn[:, lo:hi, :hd] = np.nan                        # the first key/value head's keys
+        y = backend.attention(q, kn, v, None, hd, nh, nkv)
+        cut = nh // nkv * hd
+        assert np.all(np.isnan(y[..., :cut])) and np.all(np.isfinite(y[..., cut:])), (lo, hi)
+        mask = np.zeros(Tk, np.float32)
+        mask[lo:hi] = np.nan
+        assert np.all(np.isnan(backend.attention(q, k, v, mask, hd, nh, nkv))), (lo, hi)
+
+
+@pytest.mark.parametrize("case", TILE_HD + [(1, 4, 300, 32, 4, 4), (1, 4, 300, 64, 8, 2), (1, 4, 300, 128, 4, 2)])
+def test_attention_masked_values(backend, case):
+    """Values behind masked positions: a range's leading 64s of masked positions are
+    left out whatever they hold; any other masked inf or NaN gives 0 * inf = NaN,
+    as the reference's sum does.  Also on the one-wave-per-row kernel (4 queries)."""
+    assert _attention_kernel(backend, case) == ("attention_wave" if case[1] == 4 else "attention_tile")
+    B, S, Tk, hd, nh, nkv = case
+    q, k, v = (_rand(50 + i, (B, n, h * hd)) for i, n, h in ((0, S, nh), (1, Tk, nkv), (2, Tk, nkv)))
+    mask = np.zeros(Tk, np.float32)
+    mask[:64] = -np.inf
+    vn = v.copy()
+    vn[:, 3] = np.inf
+    vn[:, 63] = np.nan
+    # rtol, atol as in test_attention_tiles
+    np.testing.assert_allclose(backend.attention(q, k, vn, mask, hd, nh, nkv),
+                               R.attention(q, k, v, mask, hd, nh, nkv), rtol=1e-4, atol=1e-5)
+    mask[63] = 0.0                                        # one position of the first 64 attended
+    vn[:, 63] = 1.0
+    assert np.all(np.isnan(backend.attention(q, k, vn, mask, hd, nh, nkv)))
+    mask[:] = 0.0
+    mask[200:232] = -np.inf
+    assert np.all(np.isfinite(backend.attention(q, k, v, mask, hd, nh, nkv)))
+    v[:, 210] = -np.inf
+    assert np.all(np.isnan(backend.attention(q, k, v, mask, hd, nh, nkv)))
 
 
 def test_attention_masks(backend):

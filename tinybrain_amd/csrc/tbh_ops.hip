@@ -866,6 +866,12 @@ __global__ __launch_bounds__(512, HD == 128 ? 2 : 4) void attention_tile(const T
 #pragma unroll
     for (int i = 0; i < NH * VW; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 
+    // Every position so far is masked (uniform): attention_wave leaves a range's
+    // leading 64s of masked positions out, and no others, so that a masked value
+    // of inf or NaN behind them gives 0 * inf = NaN there as here.  By the mask
+    // alone: a NaN score is no masked one, and fmaxf drops it.
+    bool lead = a.mask != nullptr;
+
     fetch(c0);
     stage(0);
     __syncthreads();
@@ -874,7 +880,8 @@ __global__ __launch_bounds__(512, HD == 128 ? 2 : 4) void attention_tile(const T
         const bool more = p0 + POS < c1;
         if (more) fetch(p0 + POS);
         const int64_t w0 = p0 + ks * 16 * PT;       // this wave's first position
-        if (live && w0 < c1) {
+        if (lead && (p0 - c0) % 64 == 0) lead = __all(a.mask[min(p0 + lane, c1 - 1)] == -INFINITY);
+        if (live && w0 < c1 && !lead) {
             const float *kt = &lds[buf][0][ks * 16 * PT * LD], *vt = &lds[buf][1][ks * 16 * PT * LD];
             f32x4 mk[PT], s[PT][HD / 16];
             if (a.mask)
@@ -922,43 +929,41 @@ __global__ __launch_bounds__(512, HD == 128 ? 2 : 4) void attention_tile(const T
                 for (int i = 0; i < 4; ++i) nm = fmaxf(nm, s[t][0][i]);
             nm = fmaxf(nm, __shfl_xor(nm, 16));
             nm = fmaxf(nm, __shfl_xor(nm, 32));
-            if (__any(nm != -INFINITY)) {           // else every position so far is masked
-                const float ref = nm == -INFINITY ? 0.0f : nm;
-                const float corr = expf(m - ref);
-                m = nm;
-                l *= corr;
+            const float ref = nm == -INFINITY ? 0.0f : nm;
+            const float corr = expf(m - ref);
+            m = nm;
+            l *= corr;
 #pragma unroll
-                for (int t = 0; t < PT; ++t)
+            for (int t = 0; t < PT; ++t)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        s[t][0][i] = expf(s[t][0][i] - ref);
-                        l += s[t][0][i];
-                    }
-                // sums of eight positions, added up before they join the running one
-                f32x4 pv[2 * PT][NH * VW];
-#pragma unroll
-                for (int t = 0; t < PT; ++t)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i)
-#pragma unroll
-                        for (int h = 0; h < NH; ++h) {
-                            const float *vp = &vt[(16 * t + 4 * gg + i) * LD + 64 * h + VW * n];
-                            float vv[VW];
-                            __builtin_memcpy(vv, __builtin_assume_aligned(vp, 4 * VW), sizeof vv);
-#pragma unroll
-                            for (int c = 0; c < VW; ++c) {
-                                f32x4 &d = pv[2 * t + i / 2][h * VW + c];
-                                d = __builtin_amdgcn_mfma_f32_16x16x4f32(
-                                    vv[c], s[t][0][i], i % 2 ? d : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-                            }
-                        }
-#pragma unroll
-                for (int x = 0; x < NH * VW; ++x) {
-                    f32x4 sum = pv[0][x] + pv[1][x];
-                    if constexpr (PT == 2) sum += pv[2][x] + pv[3][x];
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) o[x][i] = o[x][i] * corr + sum[i];
+                for (int i = 0; i < 4; ++i) {
+                    s[t][0][i] = expf(s[t][0][i] - ref);
+                    l += s[t][0][i];
                 }
+            // sums of eight positions, added up before they join the running one
+            f32x4 pv[2 * PT][NH * VW];
+#pragma unroll
+            for (int t = 0; t < PT; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int h = 0; h < NH; ++h) {
+                        const float *vp = &vt[(16 * t + 4 * gg + i) * LD + 64 * h + VW * n];
+                        float vv[VW];
+                        __builtin_memcpy(vv, __builtin_assume_aligned(vp, 4 * VW), sizeof vv);
+#pragma unroll
+                        for (int c = 0; c < VW; ++c) {
+                            f32x4 &d = pv[2 * t + i / 2][h * VW + c];
+                            d = __builtin_amdgcn_mfma_f32_16x16x4f32(
+                                vv[c], s[t][0][i], i % 2 ? d : f32x4{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                        }
+                    }
+#pragma unroll
+            for (int x = 0; x < NH * VW; ++x) {
+                f32x4 sum = pv[0][x] + pv[1][x];
+                if constexpr (PT == 2) sum += pv[2][x] + pv[3][x];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[x][i] = o[x][i] * corr + sum[i];
             }
         }
         if (more) stage(buf ^ 1);
