@@ -150,23 +150,40 @@ def test_attention(backend, case):
 
 # (batch, seq, kv, head_dim, heads, kv_heads): the matrix-core kernel takes 64
 # (query, query head) rows per block in groups of 16, and tiles of 32 positions
-# (64 at head_dim 32) halved between two waves; it needs 96 Ki (224 Ki at
-# head_dim 64) of (query, quad of heads, position)
+# (64 at head_dim 32) halved between two waves; which calls it takes: use_tiles
 TILE_CASES = [
-    (2, 1600, 32, 32, 1, 1),         # the fewest positions: only the first wave of each group has any
-    (2, 65, 897, 64, 2, 2),          # one row past a block; ranges over blocks, one position over
-    (2, 63, 512, 32, 3, 3),          # one row short of a block
+    (4, 1600, 32, 32, 1, 1),         # the fewest positions: only the first wave of each group has any
+    (2, 65, 897, 64, 4, 4),          # one row past a block; ranges over blocks, one position over
+    (2, 63, 1500, 32, 3, 3),         # one row short of a block
     (1, 1025, 113, 64, 4, 2),        # a last tile of one position past the first wave's half
     (1, 80, 321, 128, 4, 4),         # rows end on a group of 16
     (2, 33, 1000, 64, 16, 2),        # eight query heads per key/value head, ranges merged
     (1, 50, 1000, 128, 24, 2),       # twelve query heads per key/value head, ranges
     (1, 300, 513, 32, 12, 12),
     (1, 16, 6144, 128, 1, 1),        # the fewest rows: three groups of 16 empty
-    (1, 16, 6143, 128, 1, 1),        # just below the line: the one-wave-per-row kernel
+]
+# below the line in (query, quad of heads, position), or above it where the
+# one-wave-per-row kernel takes less time: few blocks of many tiles, blocks of
+# that kernel with one busy wave
+WAVE_CASES = [
+    (1, 16, 6143, 128, 1, 1),
+    (2, 1600, 32, 32, 1, 1),
+    (2, 65, 897, 64, 2, 2),
+    (2, 63, 512, 32, 3, 3),
+    (1, 16, 4096, 32, 8, 2),
+    (1, 87, 309, 32, 16, 16),
+    (4, 202, 202, 32, 2, 1),
+    (2, 643, 235, 64, 1, 1),
 ]
 
 
-@pytest.mark.parametrize("case", TILE_CASES)
+@pytest.mark.parametrize("case", TILE_CASES + WAVE_CASES)
+def test_attention_kernel_choice(backend, case):
+    if backend.cu_count == 256:
+        assert _attention_kernel(backend, case) == ("attention_tile" if case in TILE_CASES else "attention_wave")
+
+
+@pytest.mark.parametrize("case", TILE_CASES + WAVE_CASES)
 @pytest.mark.parametrize("masked", [False, True])
 def test_attention_tiles(backend, case, masked):
     B, S, Tk, hd, nh, nkv = case
@@ -198,19 +215,18 @@ def test_attention_tiles_special_values(backend):
     assert np.all(np.isnan(y[3, :hd])) and not np.any(np.isnan(np.delete(y, 3, 0)))
 
 
-def _attention_kernel(backend, case, aligned=True):
+def _attention_kernel(backend, case):
     """The first kernel that an attention call of this shape launches."""
     import torch
 
     B, S, Tk, hd, nh, nkv = case
-    q, k, v, out = (torch.zeros(n, device="cuda") for n in (B * S * nh * hd, B * Tk * nkv * hd,
-                                                           B * Tk * nkv * hd + 1, B * S * nh * hd))
+    q, k, v, out = (torch.zeros(B * n, device="cuda") for n in (S * nh * hd, Tk * nkv * hd, Tk * nkv * hd, S * nh * hd))
     sh, s = _abi.AttentionShape(B, S, Tk, hd, nh, nkv), torch.cuda.Stream()
-    ptr = [q.data_ptr(), k.data_ptr(), v.data_ptr() + (0 if aligned else 4)]
     torch.cuda.synchronize()
 
     def call():
-        assert backend._lib.tbh_attention_device(backend._dev, ctypes.byref(sh), *ptr, None, out.data_ptr(),
+        assert backend._lib.tbh_attention_device(backend._dev, ctypes.byref(sh), q.data_ptr(), k.data_ptr(),
+                                                 v.data_ptr(), None, out.data_ptr(),
                                                  ctypes.c_void_p(s.cuda_stream)) == _abi.OK
     call()                                                # its workspace
     torch.cuda.synchronize()

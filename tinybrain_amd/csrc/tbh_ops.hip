@@ -1197,31 +1197,77 @@ hipError_t launch_act(const tbh_device *dev, const float *x, int64_t n, float *y
 
 hipError_t launch_attention_rows(const AttnArgs &a, hipStream_t s);
 
+// Positions per range of attention_wave / attention_group (a multiple of 64, or
+// all of them) for blocks of `per_split` a range.
+int64_t wave_chunk(int64_t per_split, int64_t kv_len, int64_t cus) {
+    const int64_t target = 2 * cus;
+    if (per_split >= target || kv_len <= 64) return std::max<int64_t>(kv_len, 1);
+    const int64_t want =
+        std::min<int64_t>(std::min((target + per_split - 1) / per_split, (kv_len + 63) / 64), 1024);
+    return ((kv_len + want - 1) / want + 63) / 64 * 64;
+}
+
+// The same for attention_tile: one block per CU (eight waves), each with at
+// least 128 positions.
+int64_t tile_chunk(const TileArgs &ta, int64_t cus) {
+    const int64_t kv_len = ta.g.a.kv_len;
+    const int64_t want = std::min<int64_t>(std::min(cus / (ta.rtiles * ta.heads), kv_len / 128), 64);
+    return want > 1 ? ((kv_len + want - 1) / want + 63) / 64 * 64 : kv_len;
+}
+
 // Whether a call's rows go to attention_tile: at least one full group of 16 per
 // key/value head (so no single query of up to 15 heads per key/value head,
-// where a group's matrix work is mostly padding), and enough (block, position)
+// where a group's matrix work is mostly padding), enough (block, position)
 // pairs of attention_wave that its reads of every key and value row for each
-// of them outweigh the tile kernel's start and merge.  us, attention_wave /
+// of them outweigh the tile kernel's start and merge (us, attention_wave /
 // attention_tile, below and above the line: HD 64, 16 x 1000 positions of 32
-// heads on 4 (125 Ki) 17.6 / 20.0, of 12 on 12 (188 Ki) 17.1 / 18.8, 64 x 512
-// of 32 on 4 (256 Ki) 24.9 / 16.5; HD 32, 64 x 512 of 8 on 2 (64 Ki) 10.2 /
-// 11.0, 100 x 700 (137 Ki) 15.1 / 13.2; HD 128, 64 x 64 of 32 on 8 (32 Ki)
-// 11.6 / 12.8, 16 x 1000 (125 Ki) 36.8 / 28.5.
-bool use_tiles(const TileArgs &ta, int64_t wave_blocks) {
-    const GrpArgs &g = ta.g;
-    return ta.nrows >= 16 && g.a.kv_len >= 32 &&
-           wave_blocks * g.a.kv_len >= (g.a.hd == 64 ? 224 : 96) * 1024;
+// heads on 4 (125 Ki) 17.6 / 20.0, 64 x 512 of 32 on 4 (256 Ki) 24.9 / 16.5; HD
+// 32, 64 x 512 of 8 on 2 (64 Ki) 10.2 / 11.0, 100 x 700 (137 Ki) 15.1 / 13.2; HD
+// 128, 64 x 64 of 32 on 8 (32 Ki) 11.6 / 12.8, 16 x 1000 (125 Ki) 36.8 / 28.5),
+// and, at HD 32 and 64, less expected time.  The pairs alone sent calls to the
+// tile kernel whose few blocks each walk many tiles, or whose attention_wave
+// blocks hold one busy wave: HD 32, 16 x 4096 of 8 on 2 11.7 / 17.5, 87 x 309 of
+// 16 on 16 8.8 / 13.3, 4 x 202 x 202 of 2 on 1 8.0 / 12.3; HD 64, 2 x 643 x 235 of
+// 1 on 1 15.1 / 19.8.
+// Expected times in us: attention_wave a start, per 64-position pass (a wave's
+// latency; per 1000 passes of a block; of a wave) and the second launch of
+// several ranges; attention_tile a start, per tile (latency; per further block
+// a CU) and the merge with its part per range.  Least-squares fits over 253 and
+// 232 calls of both kernels (4 .. 1024 queries, 32 .. 4096 positions, batches 1 ..
+// 16), standard deviation 6-11 %: the calls sent to the tile kernel take at
+// most 1.13 (HD 64: 1.0) times attention_wave's time, where the pairs alone took
+// up to 1.6 (1.47).  At HD 128 none of 213 was slower there.
+bool use_tiles(const TileArgs &ta, int64_t wave_blocks, int64_t cus) {
+    const AttnArgs &a = ta.g.a;
+    if (ta.nrows < 16 || a.kv_len < 32 || wave_blocks * a.kv_len < (a.hd == 64 ? 224 : 96) * 1024) return false;
+    if (a.hd == 128) return true;
+    static constexpr struct {
+        double start, pass, block, wave, combine;
+    } kWave[2] = {{3.70, 0.20, 0.184, 0.50, 4.25}, {3.64, 0.40, 0.418, 1.29, 3.83}};
+    static constexpr struct {
+        double start, tile, further, merge, range;
+    } kTile[2] = {{4.15, 2.14, 2.75, 2.44, 0.197}, {4.89, 1.97, 2.55, 2.10, 0.198}};
+    const auto &w = kWave[a.hd == 64];
+    const auto &t = kTile[a.hd == 64];
+    const int64_t wc = wave_chunk(wave_blocks, a.kv_len, cus), ws = (a.kv_len + wc - 1) / wc;
+    const double passes = (double)((wc + 63) / 64);
+    const double wave_us = w.start + (ws > 1 ? w.combine : 0.0) +
+                           passes * (w.pass + 1e-3 * (double)ws * (w.block * (double)wave_blocks +
+                                                                   w.wave * (double)a.rows));
+    const int64_t tc = tile_chunk(ta, cus), ts = (a.kv_len + tc - 1) / tc, pos = a.hd == 32 ? 64 : 32;
+    const double further = std::max(0.0, (double)(ta.rtiles * ta.heads * ts) / (double)cus - 1.0);
+    const double tile_us = t.start + (ts > 1 ? t.merge + t.range * (double)ts : 0.0) +
+                           (double)((tc + pos - 1) / pos) * (t.tile + t.further * further);
+    return tile_us < wave_us;
 }
 
 template <int HD>
 hipError_t launch_attention_tile(tbh_device *dev, TileArgs &ta, hipStream_t s) {
     GrpArgs &g = ta.g;
     const AttnArgs &a = g.a;
-    const int64_t tiles = ta.rtiles * ta.heads, cus = std::max(1, dev->cu_count);
-    // one block per CU (eight waves), each with at least 128 positions
-    const int64_t want = std::min<int64_t>(std::min(cus / tiles, a.kv_len / 128), 64);
-    if (want > 1) {
-        g.chunk = ((a.kv_len + want - 1) / want + 63) / 64 * 64;
+    const int64_t tiles = ta.rtiles * ta.heads;
+    g.chunk = tile_chunk(ta, std::max(1, dev->cu_count));
+    if (g.chunk < a.kv_len) {
         g.splits = (int32_t)((a.kv_len + g.chunk - 1) / g.chunk);
         ta.sums = (2 * a.rows * g.splits + 3) / 4 * 4;
         const size_t bytes = (size_t)(ta.sums + a.rows * g.splits * HD) * sizeof(float);
@@ -1248,7 +1294,7 @@ hipError_t launch_attention(tbh_device *dev, const AttnArgs &a, hipStream_t s) {
     g.hchunks = (g.rep + kGrpHeads - 1) / kGrpHeads;
     g.units = (a.rows / a.nh) * a.nkv * g.hchunks;
     g.splits = 1;
-    g.chunk = std::max<int64_t>(a.kv_len, 1);
+    const int64_t cus = std::max(1, dev->cu_count);
     const bool wave = a.hd == 16 || a.hd == 32 || a.hd == 64 || a.hd == 128;
     // blocks per split: (query row, KV head, 4 query heads) for attention_wave,
     // (query row, KV head, 8 query heads) for attention_group
@@ -1259,7 +1305,7 @@ hipError_t launch_attention(tbh_device *dev, const AttnArgs &a, hipStream_t s) {
         ta.rtiles = (ta.nrows + 63) / 64;
         ta.heads = a.rows / a.nh / std::max<int64_t>(a.seq_len, 1) * a.nkv;
         ta.g = g;
-        if (use_tiles(ta, per_split)) {
+        if (use_tiles(ta, per_split, cus)) {
             switch (a.hd) {
             case 32: return launch_attention_tile<32>(dev, ta, s);
             case 64: return launch_attention_tile<64>(dev, ta, s);
@@ -1267,13 +1313,8 @@ hipError_t launch_attention(tbh_device *dev, const AttnArgs &a, hipStream_t s) {
             }
         }
     }
-    const int64_t target = 2 * (int64_t)std::max(1, dev->cu_count);
-    if (per_split < target && a.kv_len > 64) {
-        const int64_t want =
-            std::min<int64_t>(std::min((target + per_split - 1) / per_split, (a.kv_len + 63) / 64), 1024);
-        g.chunk = ((a.kv_len + want - 1) / want + 63) / 64 * 64;
-        g.splits = (int32_t)((a.kv_len + g.chunk - 1) / g.chunk);
-    }
+    g.chunk = wave_chunk(per_split, a.kv_len, cus);
+    g.splits = (int32_t)std::max<int64_t>((a.kv_len + g.chunk - 1) / g.chunk, 1);
     if (g.splits > 1) {
         const size_t bytes = (size_t)(g.units * g.splits * (2 * kGrpHeads + kGrpHeads * a.hd)) * sizeof(float);
         g.part = (float *)stream_workspace(dev, s, bytes);
