@@ -154,3 +154,38 @@ def test_pieces_in_parts(backend, kind, K, M):
     z = backend.matmul_device_noalloc(x, w, out=torch.empty_like(y))
     torch.cuda.synchronize()
     assert torch.equal(z.view(torch.int32), y.view(torch.int32))
+
+
+def _kernels(backend, kind, K, N, M, bf16):
+    """Names of the kernels of one call on a weight of random bytes, the last
+    stretch of them (its GEMM, or the last GEMV launch)."""
+    import torch
+
+    rng = np.random.default_rng(K + N)
+    if kind == "int8":
+        pq = T.QuantizedTensor((K, N), rng.integers(-127, 128, K * N, dtype=np.int8), np.full(N, 0.01, np.float32),
+                               T.QuantizationMode.perChannel)
+    else:
+        pq = T.QuantizedTensor((K, N), rng.integers(-128, 128, K * N // 2, dtype=np.int8),
+                               np.full(K * N // 32, 0.01, np.float32), T.QuantizationMode.int4,
+                               T.QuantizationPrecision.int4, 32, None, T.Layout.NK_FLAT)
+    w = T.DeviceWeight(backend, pq)
+    x = torch.zeros((M, K), dtype=torch.bfloat16 if bf16 else torch.float32, device="cuda")
+    y, stream = torch.empty((M, N), device="cuda"), torch.cuda.Stream()
+    call = lambda: (backend.matmul_bf16_device if bf16 else backend.matmul_device)(x, w, out=y, stream=stream)
+    torch.cuda.synchronize()
+    call()                                                # its workspace
+    torch.cuda.synchronize()
+    names = {n for n, _, _ in launches(call, stream)}
+    w.close()
+    return names
+
+
+# few rows of fp32 x on INT8 weights from 32 Mi elements: the GEMM from five
+# rows, from four where K is 8192 or more (mfma_min_rows)
+@pytest.mark.parametrize("K,N,M,gemv", [(2560, 14336, 4, True), (2560, 14336, 5, False), (6000, 6000, 4, True),
+                                        (8704, 4096, 4, False)])
+def test_few_rows_kernel(backend, K, N, M, gemv):
+    names = _kernels(backend, "int8", K, N, M, False)
+    assert any(n.startswith("gemv") for n in names) == gemv, names
+    assert any(n in ("gemm", "gemm_bf16") for n in names) != gemv, names

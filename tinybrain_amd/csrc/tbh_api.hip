@@ -822,9 +822,11 @@ static int64_t sgemv_min_rows(const tbh_weight &w) {
 //   INT8: 2048x2048 8 rows 7.5 / 7.9, 12 10.7 / 8.0; 4096x4096 4 rows 11.7 /
 //     12.3, 6 13.9 / 12.4; 2048x5632 4 rows 11.6 / 13.1, 6 15.3 / 12.1;
 //     5632x2048 8 rows 9.2 / 11.2 (one eight-row launch), 9 12.5 / 11.7;
-//     11008x4096 4 rows 22.3 / 20.5; 4096x11008 4 rows 48.1 / 22.0; 32000x2048
-//     4 rows 17.1 / 27.6, 6 31.6 / 25.0; 20000x1024 6 rows 11.8 / 13.6;
-//     32000x4096 4 rows 58.1 / 38.1.
+//     14336x2560 4 rows 14.4 / 17.7, 5 20.5 / 17.0; 6000x6000 4 rows 18.2 /
+//     19.6, 5 24.0 / 19.1; 11008x4096 4 rows 22.9 / 22.2, 5 24.3 / 23.4; 4096x8704
+//     4 rows 40.8 / 17.9; 4096x11008 4 rows 48.1 / 22.0; 32000x2048 4 rows 17.1 /
+//     27.6, 6 31.6 / 25.0; 20000x1024 6 rows 11.8 / 13.6; 32000x4096 4 rows 58.1 /
+//     38.1.
 //   Runtime layout (four or eight rows a launch on the VALU): 2048x2048 9
 //     rows 11.5 / 11.5; 2048x5632 4 rows 11.4 / 13.2, 6 15.5 / 13.4; 4096x4096
 //     4 rows 15.2 / 14.3; 4096x11008 4 rows 34.1 / 27.6; 11008x4096 6 rows 29.8
@@ -846,7 +848,7 @@ static int64_t mfma_min_rows(const tbh_weight &w, bool burst8) {
         if (nk < 8 * mi) return 12;
         if (wide) return nk >= 100 * mi ? 4 : nk >= 32 * mi ? 6 : 8;
         if (burst8) return 9;
-        return nk >= 32 * mi ? 4 : 6;
+        return nk < 32 * mi ? 6 : w.K >= 8192 ? 4 : 5;
     }
     return wide && nk > 24 * mi && nk < 100 * mi ? 17 : 12;
 }
