@@ -189,3 +189,13 @@ def test_few_rows_kernel(backend, K, N, M, gemv):
     names = _kernels(backend, "int8", K, N, M, False)
     assert any(n.startswith("gemv") for n in names) == gemv, names
     assert any(n in ("gemm", "gemm_bf16") for n in names) != gemv, names
+
+
+# bf16 x on INT4 K-groups of a long K: tiles of 128 x 128 that fill the CUs in
+# eight, four or (K below 4608) two parts stay on gemm_bf16 (keep_gemm_bf16)
+@pytest.mark.parametrize("K,N,M,kept", [(4096, 4096, 512, True), (4128, 1020, 2047, True), (4800, 1024, 2048, False),
+                                        (5632, 2048, 512, True), (8192, 1024, 512, True), (4096, 4096, 1024, False)])
+def test_kept_kernel(backend, K, N, M, kept):
+    names = _kernels(backend, "int4", K, N, M, True)
+    if backend.cu_count == 256:
+        assert ("gemm_bf16" in names, "gemm" in names) == (kept, not kept), names

@@ -823,18 +823,27 @@ static bool use_gemm(const tbh_weight &w, int64_t rows) {
 
 // Whether `rows` rows of bf16 x on an INT4 K-group weight stay on gemm_bf16:
 // its 128 x 128 tiles, split along K, take a long-K product of a small output
-// in one full round of blocks (32 or 64 tiles on 256 CUs), where a block's step
-// is bound by unpacking, scales and MFMA alike in both kernels and launch_gemm's
-// longer pipeline only adds its start.  us, gemm_bf16 / launch_gemm: 64 tiles
-// 2048x5632 512 rows 32.3 / 35.1, 4096x4096 256 29.8 / 32.8; 32 tiles 1024x8192 512
-// rows 27.6 / 30.6; other counts leave gemm_bf16 a part-filled round: 2048x5632
-// 333 rows 34.2 / 28.5, 1000 53.1 / 51.2, 4096x4096 333 47.5 / 35.5; and shorter or
-// larger products are launch_gemm's: 2048x2048 512 rows 22.6 / 20.3, 4096x11008
-// 256 54.3 / 50.2.
+// in one full round of blocks, where a block's step is bound by unpacking,
+// scales and MFMA alike in both kernels and launch_gemm's longer pipeline only
+// adds its start.  us, gemm_bf16 / launch_gemm on 256 CUs:
+//   64 tiles (four K parts): 2048x5632 512 rows 30.4 / 33.2, 4096x4096 256 28.7 /
+//     32.3, 1024x4096 1024 25.3 / 28.8, 1024x8192 1024 39.5 / 38.4
+//   32 tiles (eight): 1024x8192 512 rows 27.6 / 30.6, 2048x8192 256 27.7 / 30.7,
+//     1024x4096 512 19.6 / 19.5, 2048x5632 256 23.8 / 23.9
+//   128 tiles (two): K of 4096 as above (4096x4096 512 rows 37.4 / 40.2, 2048x4096
+//     1024 39.2 / 40.7, 1024x4096 2048 37.9 / 40.2), but each part's steps beyond
+//     that are slower (1024x4800 2048 47.6 / 46.5, 2048x5632 1024 46.9 / 45.8,
+//     1024x8192 2048 64.8 / 56.8)
+//   16 tiles: 2048x5632 128 rows 17.9 / 17.2, 1024x4096 256 19.1 / 14.9; 256
+//     (unsplit): 4096x4096 1024 60.3 / 55.5
+//   other counts leave a part-filled round: 2048x5632 384 rows 34.1 / 27.9,
+//     3072x4096 512 46.2 / 37.2, 1536x6144 512 40.2 / 30.3
+// Shorter or larger products are launch_gemm's: 2048x2048 512 rows 22.6 / 20.3,
+// 4096x11008 256 54.3 / 50.2.
 static bool keep_gemm_bf16(const tbh_weight &w, int64_t rows) {
     const int64_t cus = std::max(1, w.dev->cu_count), tiles = ((w.N + 127) / 128) * ((rows + 127) / 128);
     return w.path == Path::Int4KGroup && w.K >= 4096 && w.N * w.K <= (int64_t)16 << 20 &&
-           (8 * tiles == cus || 4 * tiles == cus);
+           (8 * tiles == cus || 4 * tiles == cus || (2 * tiles == cus && w.K < 4608));
 }
 
 // x [M][ldx] (fp32, or bf16) through launch_gemm, in calls whose pieces take
