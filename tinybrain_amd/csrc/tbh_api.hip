@@ -604,8 +604,7 @@ tbh_status tbh_weight_create(tbh_device *dev, const tbh_qtensor_desc *desc, tbh_
                         if (v == 0.0f || !std::isfinite(v)) continue;
                         v = std::copysign(std::max(std::ldexp(std::fabs(v), 8 - ex[(size_t)nb]), 0x1p-28f), v);
                     }
-                int64_t n_scaled = 0;
-                if (e == hipSuccess) e = upload(&w->ng_scaled, t.data(), t.size(), w->device_bytes, n_scaled);
+                if (e == hipSuccess) e = upload(&w->ng_scaled, t.data(), t.size(), w->device_bytes, w->n_ng_scaled);
                 w->stream_bytes = (count + 1) / 2 + 4 * d.n_scales;
             }
         } else {
@@ -754,7 +753,8 @@ bool weight_arrays_ok(const tbh_weight &w) {
         if (w.rows_per_nblock <= 0 || w.zp) return false;
         if (w.ng_pairs) return w.nb_half > 0 && w.n_scales_dev == 2 * (int64_t)w.nb_half * w.Kp;
         const int64_t nb = (w.Np + w.rows_per_nblock - 1) / w.rows_per_nblock;
-        return w.n_scales_dev == nb * w.Kp && w.ng_sexp && w.n_ng_sexp == nb;
+        return w.n_scales_dev == nb * w.Kp && w.ng_sexp && w.n_ng_sexp == nb && w.ng_scaled &&
+               w.n_ng_scaled == w.n_scales_dev;
     }
     return false;
 }

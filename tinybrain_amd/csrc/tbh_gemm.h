@@ -103,14 +103,16 @@ __device__ __forceinline__ i32x4 make_rsrc(const void *p, int bytes) {
 // 16 (or 4) bytes per active lane from buffer offset `off` + `soff` to LDS
 // byte lds + 16 (4) * lane; offsets past the buffer's size write zeros.  No
 // register receives the load; completion is waited for by dma_wait.  (One
-// wait state between the write of M0 and the load that reads it.)
+// wait state between the write of M0 and the load that reads it.  M0 is a
+// reserved register, which the compiler neither allocates nor takes as a
+// clobber; the built kernels use it in these statements only.)
 __device__ __forceinline__ void dma16(uint32_t lds, i32x4 r, uint32_t off, uint32_t soff) {
     asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds" ::"s"(lds), "v"(off), "s"(r),
                  "s"(soff) : "memory");
 }
 // The same from the lanes of `mask` alone, 16 or 4 bytes a lane (called with
-// every lane active, without a branch that would end the basic block the
-// surrounding instructions are scheduled in).
+// every lane active, as EXEC is left, and without a branch that would end the
+// basic block the surrounding instructions are scheduled in).
 template <int BYTES>
 __device__ __forceinline__ void dma_lanes(uint32_t lds, i32x4 r, uint32_t off, uint32_t soff, uint64_t mask) {
     if constexpr (BYTES == 16)
@@ -239,10 +241,12 @@ constexpr int step_bytes(int kind, int xp, int tm, int tn) {
 constexpr int step_bufs(int kind, int xp, int tm, int tn) {
     return 4 * step_bytes(kind, xp, tm, tn) <= 160 * 1024 ? 4 : 160 * 1024 / step_bytes(kind, xp, tm, tn);
 }
-// (runtime-layout tiles over 16 x 16 MFMA tiles per wave spill registers)
+// (runtime-layout tiles over 16 x 16 MFMA tiles per wave spill registers; its
+// 64 x 256 tile of one piece is never the cheapest: 0 of 34000 drawn products)
 constexpr bool tile_fits(int kind, int xp, int tm, int tn) {
     if (xp == 3 && (kind == W4N || tm != 4)) return false;   // few rows of x only
-    return step_bufs(kind, xp, tm, tn) >= 3 && !(kind == W4N && tm * tn > 16);
+    if (kind == W4N && (tm * tn > 16 || (xp == 1 && tm == 4 && tn == 2))) return false;
+    return step_bufs(kind, xp, tm, tn) >= 3;
 }
 
 template <int KIND, int XP, int TM, int TN>

@@ -113,8 +113,11 @@ struct tbh_weight {
     int32_t *ng_sexp = nullptr;
     int64_t n_ng_sexp = 0;
     // Int4NGroup: the scale table times 2^(8 - ng_sexp), nonzero entries at
-    // least 2^-28 in magnitude, as the prefill GEMM stages it
+    // least 2^-28 in magnitude, as the prefill GEMM stages it (the table's own
+    // size again: 4 bytes per (N-block, k), at N-blocks of 32 rows a quarter of
+    // the packed weights, and a fifth of all that the weight held before)
     float *ng_scaled = nullptr;
+    int64_t n_ng_scaled = 0;
     bool mfma_tiles = false;     // data in 1 KiB MFMA tiles (else K-contiguous rows)
 
     // generic path: the reference arrays as given
