@@ -1,18 +1,18 @@
-"""Error bounds of the two f16-piece decompositions the prefill GEMM uses
-(tbh_prefill.hip), restated in numpy and checked over random and edge-case
-values on the CPU.
+"""Error bounds of the two f16-piece decompositions of the prefill GEMM
+(tbh_gemm.h, tbh_gemm.hip), restated in numpy and checked over random and
+edge-case values on the CPU, and what the GEMM tests' bound makes of them.
 
-- x pieces (gemm_bf16 with fp32 x, gemm_ngw with fp32 x): v scaled into
-  |v| <= 2^15, hi = f16(v) and lo = f16(v - hi), both rounded to nearest:
-  |v - (hi + lo)| <= max(2^-22 |v|, 2^-25).
-- weight pieces (gemm_ngw): w scaled into |w| < 2^15, hi = w rounded toward
+- x pieces (x_pieces of fp32 x): v scaled into |v| <= 2^15, hi = f16(v) and
+  lo = f16(v - hi), both rounded to nearest: |v - (hi + lo)| <=
+  max(2^-22 |v|, 2^-25).
+- weight pieces (unpack4n): w scaled into |w| < 2^15, hi = w rounded toward
   zero, lo = lo_piece(w, w - hi) rounded to nearest, where lo_piece keeps the
   remainder at least 2^-24 in magnitude with w's sign unless w = 0:
   |w - (hi + lo)| <= max(2^-21 |w|, 2^-24), lo has w's sign, and lo = 0
   only for w = 0.  So an infinite x times the two pieces gives inf * w
   (+-inf, or NaN for w = 0) for every |w| >= 2^-24.  Below that hi would be
-  0, which is why the kernel floors a scaled scale at 2^-28 for weights
-  whose scales span that far (|16 q| >= 16 makes |w| >= 2^-24 for q != 0).
+  0, which is why scaled scales are kept at 2^-28 or more (|16 q| >= 16 makes
+  |w| >= 2^-24 for q != 0).
 """
 import numpy as np
 import pytest
@@ -111,3 +111,22 @@ def test_floored_scales_keep_the_high_piece():
         nz = w != 0
         assert np.all(nz == ((q16 != 0) & (s != 0)))
         assert np.all(hi[nz] != 0) and np.all(np.sign(hi[nz].astype(np.float32)) == np.sign(w[nz]))
+
+
+@pytest.mark.parametrize("K", [72, 512, 2048, 8192, 11008])
+def test_gemm_bound_sees_a_missing_piece(K):
+    # the bound of test_gpu_gemm.py, 8 * 2^-24 |x| |w| per output: products of
+    # the pieces keep to an eighth of it, products without x's low piece, or
+    # without the weights', do not keep to it
+    rng = np.random.default_rng(K)
+    x = rng.normal(size=(32, K)).astype(np.float32) * np.float32(2.0 ** 12)    # under 2^15
+    w = rng.normal(size=(K, 32)).astype(np.float32) * np.float32(2.0 ** 12)
+    (xh, xl), (wh, wl) = ([p.astype(np.float64) for p in f(v)] for f, v in ((_x_pieces, x), (_w_pieces, w)))
+    x64, w64 = x.astype(np.float64), w.astype(np.float64)
+    P = np.linalg.norm(x64, axis=1)[:, None] * np.linalg.norm(w64, axis=0)
+
+    def worst(y):
+        return np.max(np.abs(y - x64 @ w64) / P) * 2.0 ** 24
+
+    assert worst((xh + xl) @ w64) <= 1 and worst((xh + xl) @ (wh + wl)) <= 1
+    assert worst(xh @ w64) > 8 and worst((xh + xl) @ wh) > 8

@@ -15,6 +15,7 @@ import pytest
 
 import oracle as O
 import tinybrain_amd as T
+from launches import gemms, launches
 from tinybrain_amd import _abi
 
 pytestmark = pytest.mark.gpu
@@ -895,26 +896,43 @@ def test_prefill_bf16(backend, prec, K, N, M):
     _prefill_check(backend, pq, oq, M, seed=5 + M)
 
 
-# Tile counts that fill whole rounds of resident blocks and leave at most
-# half a tile's time for a last round once its tiles are split along K: the
-# leftover tiles' parts are summed by a second launch (INT8 128 x 128 blocks:
-# two per CU, 512 at once; INT4: one per CU, 256).  Ragged N puts split tiles
-# on the output's edge.  INT8 M = 2048 (704 tiles, 192 left) stays unsplit:
-# its 192 tiles already have a CU each.
+def _prefill_launches(backend, pq, M):
+    """Kernels of one bf16 call of M rows, workspace at hand."""
+    import torch
+
+    K, N = pq.shape
+    x, y = torch.zeros((M, K), dtype=torch.bfloat16, device="cuda"), torch.empty((M, N), device="cuda")
+    w, s = backend.weight(pq), torch.cuda.Stream()
+    torch.cuda.synchronize()
+    backend.matmul_bf16_device(x, w, out=y, stream=s)
+    torch.cuda.synchronize()
+    return launches(lambda: backend.matmul_bf16_device(x, w, out=y, stream=s), s)
+
+
+# Tile counts that leave a few tiles for a last round of blocks: those are
+# split along K, their parts summed by a second launch (256 CUs; ragged M puts
+# split tiles on the output's edge).
 @pytest.mark.parametrize("prec,K,N,M", [
-    ("int8", 2048, 5632, 1536),   # 528 tiles: 16 left, 8 parts
-    ("int8", 2048, 5000, 2048),   # 640 tiles: 128 left, 2 parts, the last N tile ragged
-    ("int8", 1000, 5632, 3072),   # 1056 tiles: 32 left; K of 16 steps, 8 parts of 2
-    ("int4", 5632, 2048, 3072),   # 384 tiles: 128 left after one round of 256, 2 parts
-    ("int8", 2048, 5632, 2048),   # unsplit
+    ("int8", 4096, 11008, 322),   # 258 tiles of 128 x 128: 2 left, 8 parts
+    ("int8", 2048, 5632, 322),    # 264 of 64 x 128: 8 left, 8 parts
+    ("int8", 5632, 2048, 1098),   # 288 of 64 x 128: 32 left, 8 parts
+    ("int4", 2048, 5632, 400),    # 308 of 64 x 128: 52 left, 4 parts
+    ("int4", 2048, 5632, 1100),   # 264 of 192 x 128: 8 left, 8 parts
+    ("int4_rt", 4096, 11008, 322),  # 258 of 128 x 128: 2 left, 8 parts
+    ("int8", 2048, 5632, 2048),   # 242 tiles, unsplit
 ])
 def test_prefill_split_tail(backend, prec, K, N, M):
     if prec == "int8":
         oq = _int8_pc(71 + K + M, K, N)
         pq = _product(oq, (K, N))
-    else:
+    elif prec == "int4":
         oq = _int4_nk(73 + K + M, K, N, 32)
         pq = _product(oq, (K, N), T.Layout.NK_FLAT)
+    else:
+        oq = _int4_kn(79 + K + M, K, N, 32)
+        pq = _product(oq, (K, N))
+    if backend.cu_count == 256:
+        assert _prefill_launches(backend, pq, M)[-1].name == ("gemm" if M == 2048 else "tail_sum")
     _prefill_check(backend, pq, oq, M, seed=9 + M)
 
 
@@ -924,10 +942,11 @@ def test_prefill_split_tail_graph(backend):
     # for bit
     import torch
 
-    K, N, M = 2048, 5632, 1536
+    K, N, M = 2048, 5632, 322
     oq = _int8_pc(201, K, N)
     pq = _product(oq, (K, N))
     w = backend.weight(pq)
+    assert backend.cu_count != 256 or _prefill_launches(backend, pq, M)[-1].name == "tail_sum"
     x = torch.from_numpy(O.fill_normal(202, M * K).reshape(M, K)).to(torch.bfloat16).cuda()
     s = torch.cuda.Stream()
     y = torch.empty((M, N), dtype=torch.float32, device="cuda")
@@ -951,58 +970,22 @@ def test_prefill_split_tail_graph(backend):
     del g
 
 
-def _prefill_tile(prec, N, M, K=0, cus=256):
-    """The launch rule of tbh_prefill.hip (launch_prec) for bf16 x, restated
-    to show which tile family and wave count each case below reaches."""
-    Np = -(-N // 8) * 8
-    t128 = -(-Np // 128) * -(-M // 128)
-    t64x128 = -(-Np // 128) * -(-M // 64)
-    t64 = -(-Np // 64) * -(-M // 64)
-    if M >= 256:
-        if t128 >= cus:
-            return "128x128", 8
-        if t64 >= 2 * cus and (prec == "int8" or -(-K // 64) <= 48):
-            return "64x64", 4
-        return "128x128 split", 8
-    if prec == "int4":
-        return "64x128 split", 8
-    if t128 >= cus:
-        return "128x128", 4
-    if t64x128 >= cus:
-        return "64x128", 4
-    return "64x64 split", 4
-
-
-@pytest.mark.parametrize("K,N,M,tile", [
-    (2048, 5632, 2048, ("128x128", 8)),      # BASELINE configs[3] INT8 at M = 2048
-    (2048, 5632, 128, ("64x64 split", 4)),   # configs[3] INT8 at M = 128
-    (2048, 32000, 129, ("128x128", 4)),      # 4-wave 128 x 128, ragged M
-    (2048, 20480, 128, ("64x128", 4)),       # 64 x 128
-    (4096, 520, 300, ("128x128 split", 8)),  # 8-wave 128 x 128 split along K, ragged N
+@pytest.mark.parametrize("prec,K,N,M,tile", [
+    ("int8", 2048, 5632, 2048, (12, 2)),
+    ("int8", 2048, 5632, 128, (4, 1)),
+    ("int8", 2048, 32000, 129, (12, 1)),   # ragged M: a third of the tile rows empty
+    ("int8", 2048, 20480, 128, (8, 1)),
+    ("int8", 4096, 520, 300, (4, 1)),      # split along K, ragged N
+    ("int4", 2048, 5632, 512, (8, 1)),
+    ("int4", 5632, 2048, 1024, (8, 1)),    # split along K
 ])
-def test_prefill_bf16_int8_tiles(backend, K, N, M, tile):
-    # every INT8 tile family of the prefill launch rule under parity
-    assert backend.cu_count != 256 or _prefill_tile("int8", N, M) == tile
-    oq = _int8_pc(131 + K + N + M, K, N)
-    _prefill_check(backend, _product(oq, (K, N)), oq, M, seed=29 + M)
-
-
-def test_prefill_bf16_int4_64x64(backend):
-    # INT4 on 64 x 64 tiles without a K split (M >= 256, too few 128 x 128
-    # tiles for the CUs, enough 64 x 64 tiles for two per CU, short rows)
-    K, N, M = 2048, 5632, 512
-    assert backend.cu_count != 256 or _prefill_tile("int4", N, M, K) == ("64x64", 4)
-    oq = _int4_nk(137, K, N, 32)
-    _prefill_check(backend, _product(oq, (K, N), T.Layout.NK_FLAT), oq, M, seed=31)
-
-
-def test_prefill_bf16_int4_128x128_split(backend):
-    # INT4 with rows of more than 48 K steps where the same tile counts
-    # would give INT8 64 x 64 tiles: 128 x 128 tiles split along K
-    K, N, M = 5632, 2048, 1024
-    assert backend.cu_count != 256 or _prefill_tile("int4", N, M, K) == ("128x128 split", 8)
-    oq = _int4_nk(137, K, N, 32)
-    _prefill_check(backend, _product(oq, (K, N), T.Layout.NK_FLAT), oq, M, seed=31)
+def test_prefill_bf16_tiles(backend, prec, K, N, M, tile):
+    # tiles of (16 rows, 128 columns) on 256 CUs
+    oq = _int8_pc(131 + K + N + M, K, N) if prec == "int8" else _int4_nk(137, K, N, 32)
+    pq = _product(oq, (K, N), T.Layout.KN_FLAT if prec == "int8" else T.Layout.NK_FLAT)
+    if backend.cu_count == 256:
+        assert [(g.tm, g.tn) for g in gemms(_prefill_launches(backend, pq, M))] == [tile]
+    _prefill_check(backend, pq, oq, M, seed=29 + M)
 
 
 def test_prefill_bf16_large_m(backend):
@@ -1012,9 +995,8 @@ def test_prefill_bf16_large_m(backend):
 
 
 def test_prefill_bf16_int4_k128_steps(backend):
-    # INT4 with every CU holding a 128 x 128 tile (16 x 16 tiles on 256 CUs)
-    # stages K steps of 128: ragged M and N, K = 1056 ending in a partial
-    # step (1056 = 8 * 128 + 32), zero points
+    # INT4 with a tile of every size for every CU: ragged M and N, K = 1056
+    # ending in half a step, zero points
     K, N, M = 1056, 2000, 2000
     q4 = _int4_nk(89, K, N, 32)
     q4.zero_points = ((np.arange(q4.scales.size) % 5) - 2).astype(np.int8)
