@@ -372,6 +372,8 @@ def measure_prefill(args, backend, T, torch, workload, cpu_budget):
     tbh_matmul_bf16_device calls over a >= 2 GiB weight pool) or PREFILL_F32
     workload (tbh_matmul_device with fp32 x).  Returns the result object (the
     bench line's fields)."""
+    from tinybrain_amd._launches import launches
+
     f32 = workload in PREFILL_F32
     prec, gs, (N, K), M = (PREFILL_F32 if f32 else PREFILL)[workload]
     matmul = backend.matmul_device if f32 else backend.matmul_bf16_device
@@ -444,7 +446,7 @@ def measure_prefill(args, backend, T, torch, workload, cpu_budget):
     roof["frac"] = round(roof["achieved"] / roof["peak"], 4)
     # past 64 rows the f16 forms: runtime-layout INT4, fp32 x as two f16 pieces
     f16 = M > 64 and (prec == "int4kn" or f32)
-    kern = "gemm_bf16" if M <= 64 and (f32 or prec == "int4kn") else "gemm"
+    kern = next(n for n, _, _ in launches(lambda: step(0), cap) if "gem" in n)   # gemm, gemm_bf16 or a GEMV
     x_form = ("fp32 x, two f16 pieces" if f16 else "fp32 x, three bf16 pieces") if f32 else "bf16 x"
     roof.update({"traffic": profiled_traffic(prec, N, K, M, "prefill_f32" if f32 else "prefill"),
                  "kernel": f"{kern} {N}x{K} M={M} ({pool[0].path}, {x_form})",

@@ -15,7 +15,7 @@ import numpy as np
 import pytest
 
 import oracle as O
-from launches import gemms, launches
+from tinybrain_amd._launches import gemms, launches
 from tinybrain_amd import _abi
 import tinybrain_amd as T
 from test_gpu_sweep import _oracle_weight, _weight
@@ -257,6 +257,22 @@ def test_small_scratch_same_bits(backend, kind, K, N, M):
             backend.set_option(_abi.OPT_NOALLOC_SCRATCH_BYTES, 0)
         assert torch.equal(y.view(torch.int32), ref.view(torch.int32)), (kind, K, N, M, limit)
     _check(ref, x, _oracle_weight(qt, pq.layout), (kind, K, N, M))
+
+
+@pytest.mark.parametrize("kind", ["int8", "int4_nk_g32_zp"])
+def test_rows_too_long(backend, kind):
+    """K from 2^20 runs on the register-staged GEMM (buffer offsets of the other
+    would pass 2^30)."""
+    import torch
+
+    K, N, M = 1 << 20, 24, 3
+    qt, pq = _weight(kind, K, N, seed=11)
+    w, W = T.DeviceWeight(backend, pq), _oracle_weight(qt, pq.layout)
+    x, y = torch.from_numpy(O.fill_normal(31, M * K).reshape(M, K)).cuda(), torch.empty((M, N), device="cuda")
+    for xi in (x, x.to(torch.bfloat16)):
+        assert _tile_launches(backend, xi, w, y)[0].name == "gemm_bf16"
+        _check(y, xi, W, (kind, K, N, M, xi.dtype))
+    w.close()
 
 
 # fp32 x of long prompts, whose pieces pass 128 MiB and are made in parts: 4096

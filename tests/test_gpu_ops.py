@@ -12,7 +12,7 @@ import numpy as np
 import pytest
 
 import tinybrain_amd as T
-from launches import launches
+from tinybrain_amd._launches import launches
 from oracle import ops_ref as R
 from tinybrain_amd import _abi
 from tinybrain_amd.quantized import PreconditionFailure

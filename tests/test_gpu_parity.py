@@ -15,7 +15,7 @@ import pytest
 
 import oracle as O
 import tinybrain_amd as T
-from launches import gemms, launches
+from tinybrain_amd._launches import gemms, launches
 from tinybrain_amd import _abi
 
 pytestmark = pytest.mark.gpu

@@ -1,5 +1,5 @@
-"""The kernels that one call enqueues, read from a captured HIP graph, so that a
-test can say which kernel and tile its case ran."""
+"""The kernels that one call enqueues, read from a captured HIP graph, so that
+tests and the benchmark can say which kernel and tile a case ran."""
 import ctypes
 import re
 from collections import namedtuple

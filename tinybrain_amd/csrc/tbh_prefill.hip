@@ -1,7 +1,9 @@
-// tbh_prefill.hip -- the prefill route (M >= 64 rows of bf16 x, and fp32 x from
-// a per-weight row count): the GEMM of tbh_gemm.h past 64 rows and on larger
-// weights, and the register-staged bf16 MFMA GEMM here, gemm_bf16, for the
-// rest (use_gemm, keep_gemm_bf16).
+// tbh_prefill.hip -- the prefill route (bf16 x of any row count, and fp32 x
+// from a per-weight row count): the GEMM of tbh_gemm.h, and the
+// register-staged bf16 MFMA GEMM here, gemm_bf16, for few rows of fp32 x or of
+// runtime-layout INT4 (use_gemm), for products of few full tiles
+// (keep_gemm_bf16) and where the other has no scratch (capture) or rows too
+// long for it (gemm_supported).
 //
 // y[M, N] = x[M, K] (bf16) . dequantize(W)[K, N], fp32 accumulation, for the
 // repacked K-contiguous row layout.  This is the one dense contraction of the
@@ -13,9 +15,10 @@
 // A block of four or eight waves owns a BM x BN output tile; its waves, as
 // 2 x (waves / 2), own (BM/2) x (BN/(waves/2)) each, as TM x TN tiles of
 // v_mfma_f32_16x16x32_bf16 (eight waves: two per SIMD from one block).  Per
-// K step of 64 (128 for unsplit INT4 128 x 128 tiles) the block stages x
-// (bf16, as given) and the dequantized weight tile in LDS; global loads of
-// step t+1 are in flight while step t's MFMAs run.  Weight operands are exact:
+// K step of 64 (128 for unsplit INT4 128 x 128 tiles of fp32 x) the block
+// stages x (bf16, as given, or its pieces) and the dequantized weight tile in
+// LDS; global loads of step t+1 are in flight while step t's MFMAs run.  Weight
+// operands are exact:
 //   * INT8 (one scale per row): q - zp is an integer of magnitude <= 255,
 //     exact in bf16; the row scale multiplies the fp32 result once.
 //   * INT4 K-groups: groups are whole multiples of 32 along K, so each
@@ -30,9 +33,6 @@
 
 #include <algorithm>
 #include <cstdlib>
-#include <map>
-#include <mutex>
-#include <tuple>
 #include <type_traits>
 
 namespace tbh {
@@ -41,9 +41,6 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
-typedef float f32x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x2 __attribute__((ext_vector_type(2)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int kBK = 64;           // K per staged step (two MFMA K-steps of 32) unless a launch takes 128
 // bf16 of padding per LDS row (32 bytes): rows of 160 (K steps of 64) or 288
@@ -431,33 +428,18 @@ void gemm_bf16(const PParams p) {
     store_step(0, 0, part);
     lds_barrier();
     load_step(t_begin + 2, 0, part);
-    // INT8 with bf16 x issues a step's MFMAs before it stages the next step,
-    // so the dequantization and LDS stores run while the matrix cores work
-    // (same results bit for bit; INT8 5632x2048 M = 2048 74.4 -> 71.9 us,
-    // M = 512 30.6 -> 29.8 us).  The INT4 kernels keep staging first: in
-    // that order their register allocation spills (M = 128 17.9 -> 27.3
-    // us); so does the fp32-x form, which lost 2-3 % (M = 128 x rows 31.2 ->
-    // 32.2 us).
+    // A step is staged before the one before it is computed: the other order
+    // spills the INT4 kernels' registers (M = 128 17.9 -> 27.3 us) and the
+    // fp32-x form's (M = 128 31.2 -> 32.2 us).
     auto iteration = [&](int t0, auto full) {
-        if constexpr (PREC == 8 && XF == 0) {
-            compute(0);                    // step t0
-            store_step(1, 1, full);        // step t0 + 1
-            load_step(t0 + 3, 1, full);
-            lds_barrier();
-            compute(1);                    // step t0 + 1
-            store_step(0, 0, full);        // step t0 + 2
-            load_step(t0 + 4, 0, full);
-            lds_barrier();
-        } else {
-            store_step(1, 1, full);        // step t0 + 1
-            load_step(t0 + 3, 1, full);
-            compute(0);                    // step t0
-            lds_barrier();
-            store_step(0, 0, full);        // step t0 + 2
-            load_step(t0 + 4, 0, full);
-            compute(1);                    // step t0 + 1
-            lds_barrier();
-        }
+        store_step(1, 1, full);        // step t0 + 1
+        load_step(t0 + 3, 1, full);
+        compute(0);                    // step t0
+        lds_barrier();
+        store_step(0, 0, full);        // step t0 + 2
+        load_step(t0 + 4, 0, full);
+        compute(1);                    // step t0 + 1
+        lds_barrier();
     };
     if constexpr (kTwoForm) {
         const int t_full = n0 + BN <= p.Np ? kend / BK : 0;
@@ -591,15 +573,11 @@ hipError_t launch_tile(const PParams &p, int splits, hipStream_t s) {
             if (w8) hipLaunchKernelGGL((gemm_bf16<PREC, BM, BN, false, 8, BK, 1, 0>), grid, dim3(512), 0, s, p);
             else hipLaunchKernelGGL((gemm_bf16<PREC, BM, BN, false, 4, BK, 1, 0>), grid, dim3(256), 0, s, p);
         }
-    } else {             // bf16 x
-        const bool w8 = waves == 8 || (waves != 4 && BN == 128 && (p.M >= 256 || PREC == 4));
-        if (p.zp) {
-            if (w8) hipLaunchKernelGGL((gemm_bf16<PREC, BM, BN, true, 8, BK, 0, 0>), grid, dim3(512), 0, s, p);
-            else hipLaunchKernelGGL((gemm_bf16<PREC, BM, BN, true, 4, BK, 0, 0>), grid, dim3(256), 0, s, p);
-        } else {
-            if (w8) hipLaunchKernelGGL((gemm_bf16<PREC, BM, BN, false, 8, BK, 0, 0>), grid, dim3(512), 0, s, p);
-            else hipLaunchKernelGGL((gemm_bf16<PREC, BM, BN, false, 4, BK, 0, 0>), grid, dim3(256), 0, s, p);
-        }
+    } else if constexpr (BN == 128 && BK == kBK && (PREC == 4 || BM == 128)) {   // bf16 x
+        if (p.zp) hipLaunchKernelGGL((gemm_bf16<PREC, BM, BN, true, 8, BK, 0, 0>), grid, dim3(512), 0, s, p);
+        else hipLaunchKernelGGL((gemm_bf16<PREC, BM, BN, false, 8, BK, 0, 0>), grid, dim3(512), 0, s, p);
+    } else {
+        return hipErrorInvalidValue;   // launch_prec takes bf16 x to no other tile
     }
     return hipGetLastError();
 }
@@ -669,58 +647,53 @@ hipError_t launch_prec(const tbh_weight &w, const PParams &p, hipStream_t s, con
     const int64_t t128 = ((p.Np + 127) / 128) * ((p.M + 127) / 128);
     const int64_t t64x128 = ((p.Np + 127) / 128) * ((p.M + 63) / 64);
     const int64_t t64 = ((p.Np + 63) / 64) * ((p.M + 63) / 64);
-    static const int force = [] {   // 1: 64 x 64, 2: 64 x 128, 3: 128 x 128 tiles
+    // bf16 x, eight waves a block, split along K to a block per CU: INT4 of few
+    // full tiles (keep_gemm_bf16), 64 x 128 below 256 rows (2048x5632: M = 64
+    // 16.9 -> 14.9 us, M = 128 22.2 -> 18.5 us; 128 x 128 there 18.1 -> 20.4), and
+    // rows too long for launch_gemm
+    if (!p.xf) {
+        if constexpr (PREC == 4) {
+            if (p.M < 256) return launch_split<PREC, 64, 128>(w, p, t64x128, 1, s, scr);
+        }
+        return launch_split<PREC, 128, 128>(w, p, t128, 1, s, scr);
+    }
+    static const int force = [] {   // fp32 x: 1: 64 x 64, 2: 64 x 128, 3: 128 x 128 tiles
         const char *v = std::getenv("TBH_PREFILL_TILE");
         return v && *v ? std::atoi(v) : 0;
     }();
     if (force == 1) return launch_split<PREC, 64, 64>(w, p, t64, 2, s, scr);
     if (force == 2) return launch_split<PREC, 64, 128>(w, p, t64x128, 1, s, scr);
     if (force == 3) return launch_split<PREC, 128, 128>(w, p, t128, 1, s, scr);
+    // fp32 x, four product rows per x row: up to 64 x rows, or any number that
+    // finds no scratch for launch_gemm.
     if (p.M >= 256) {
         // Timestamps inside the kernel showed a block with one wave per SIMD
         // spending three quarters of each K step on global-load waits,
         // dequantization, LDS traffic and barriers that nothing overlaps;
         // two blocks on a CU took 1.2x the time of one.  So: 128 x 128 tiles
         // as 8-wave blocks (two waves per SIMD) when they give every CU a
-        // block; else 64 x 64 tiles when they give two blocks per CU without
-        // a K split (64 x 128 tiles never do here: there are at most twice as
-        // many as 128 x 128 tiles, which are fewer than the CUs); else 128 x
-        // 128 split along K to a block per CU.  Measured
-        // against 4-wave blocks chosen to give every CU a block: INT8
-        // 5632x2048 M = 512 35.1 -> 31 us (64 x 64), INT4 2048x5632 M = 512
-        // 52.2 -> 32.5 us (128 x 128, 4 splits), M = 2048 136 -> 89 us; INT8
-        // M = 2048 unchanged at 77 us.
+        // block; else, for INT8, 64 x 64 tiles when they give two blocks per
+        // CU without a K split (64 x 128 tiles never do here: there are at
+        // most twice as many as 128 x 128 tiles, which are fewer than the
+        // CUs); else 128 x 128 split along K to a block per CU.
         // INT4 128 x 128 tiles without a K split stage K steps of 128 (half
         // the barriers and loop trips per flop; its group scale per MFMA
-        // makes each step's VALU work larger): 2048x5632 M = 2048 90.4 ->
-        // 84.1 us.  INT8 launches measured slower with 128 (M = 512 on 64 x 64
-        // tiles 31.7 -> 33.6 us, M = 2048 79.0 -> 79.9 us), and the split INT4
-        // launch at M = 512 no faster (32.4 -> 32.8 us).
-        // INT4 takes 64 x 64 tiles only with bf16 x and short rows, else the
-        // split 128 x 128 tiles (us, 64 x 64 / 128 x 128 split: bf16 x,
-        // 5632x2048 (32 K steps) M = 512 36.0 / 41.8, 2048x5632 (88 steps) at
-        // 1024 rows 74.1 / 47.6; fp32 x in two f16 pieces, 5632x2048 M = 512
-        // 90.9 / 74.6, 2048x5632 M = 512 101.8 / 58.2).
+        // makes each step's VALU work larger: 2048x5632 at 2048 product rows
+        // 90.4 -> 84.1 us; INT8 79.0 -> 79.9).
         if (t128 >= cus)
             return PREC == 4 ? launch_split<PREC, 128, 128, 128>(w, p, t128, 1, s, scr)
                              : launch_split<PREC, 128, 128>(w, p, t128, 1, s, scr);
-        const int64_t steps64 = (p.chunks * (int64_t)(PREC == 8 ? kInt8ChunkElems : kInt4ChunkElems) + 63) / 64;
-        if (t64 >= 2 * cus && (PREC == 8 || (!p.xf && steps64 <= 48)))
-            return launch_split<PREC, 64, 64>(w, p, t64, 2, s, scr);
+        if (PREC == 8 && t64 >= 2 * cus) return launch_split<PREC, 64, 64>(w, p, t64, 2, s, scr);
         return launch_split<PREC, 128, 128>(w, p, t128, 1, s, scr);
     }
     // Fewer rows (HBM-bound).  INT4, whose K steps carry a group scale per
-    // MFMA: 64 x 128 tiles as 8-wave blocks, split along K to a block per CU
-    // (2048x5632: M = 64 16.9 -> 14.9 us, M = 128 22.2 -> 18.5 us).  INT8:
-    // the largest tile that still gives every CU a block; below that, 64 x 64
-    // tiles split along K until there are two blocks per CU (a 64 x 64 block
-    // does little work per K step, so one per CU leaves its latency exposed;
-    // 8-wave 64 x 128 tiles measured the same at M = 64 and 4 % slower at
-    // M = 128).
-    // fp32 x at 32..63 rows (128..252 product rows): 128 x 128 tiles split
-    // along K (2048x5632 at 32 rows 16.6 -> 14.8 us; bf16 x at M = 128 is
-    // slower that way, 18.1 -> 20.4 us)
-    if (PREC == 4 && p.xf && p.M >= 128) return launch_split<PREC, 128, 128>(w, p, t128, 1, s, scr);
+    // MFMA: 128 x 128 tiles from 32 x rows (2048x5632 at 32 rows 16.6 -> 14.8
+    // us), else 64 x 128, as 8-wave blocks, split along K to a block per CU.
+    // INT8: the largest tile that still gives every CU a block; below that, 64
+    // x 64 tiles split along K until there are two blocks per CU (a 64 x 64
+    // block does little work per K step, so one per CU leaves its latency
+    // exposed).
+    if (PREC == 4 && p.M >= 128) return launch_split<PREC, 128, 128>(w, p, t128, 1, s, scr);
     if (PREC == 4) return launch_split<PREC, 64, 128>(w, p, t64x128, 1, s, scr);
     if (t128 >= cus) return launch_split<PREC, 128, 128>(w, p, t128, 1, s, scr);
     if (t64x128 >= cus) return launch_split<PREC, 64, 128>(w, p, t64x128, 1, s, scr);
