@@ -146,7 +146,7 @@ tbh_status tbh_device_get_info(const tbh_device *dev, int32_t *ordinal, int32_t 
  *     device opens, sets the initial value.
  *   TBH_OPT_NOALLOC_SCRATCH_BYTES: the most scratch bytes
  *     tbh_matmul_device_noalloc may use on this device, 1 .. 16 MiB; 0 (the
- *     default) is the whole 16 MiB array.  A call needing more is rejected.
+ *     default) is the whole 16 MiB array.
  *   TBH_OPT_MFMA_MIN_ROWS: fewest rows of fp32 x that tbh_matmul* send to the
  *     MFMA GEMM (x split exactly into bf16 pieces) for every weight; 0
  *     restores the per-weight rule.
@@ -243,12 +243,14 @@ tbh_status tbh_matmul_device(const tbh_weight *w, const float *x, int64_t M,
  * allocate device memory: code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc.  Same product, same kernels, same
  * arguments; the split-K partial sums (matrix-core small-M GEMV, MFMA GEMM)
- * and the GEMM's per-row exponents of x
- * go to a fixed 16 MiB scratch array per GPU (held until the process ends)
- * instead of a per-stream workspace, and the call makes no allocation.  A
- * call one of whose launches would need more than the scratch holds (16 MiB,
- * or TBH_OPT_NOALLOC_SCRATCH_BYTES) returns TBH_E_INVALID before that launch
- * is enqueued; rows of x that an earlier launch of the same call took on a
+ * and the GEMM's 16-bit pieces of x go to a fixed 16 MiB scratch array per
+ * GPU (held until the process ends) instead of a per-stream workspace, and
+ * the call makes no allocation.  The MFMA GEMM past 64 rows, or of a larger
+ * weight, takes x and K in parts where the scratch (16 MiB, or
+ * TBH_OPT_NOALLOC_SCRATCH_BYTES) does not hold them at once, with the same
+ * bits.  A call another launch of which would need more returns TBH_E_INVALID
+ * before that launch is enqueued; rows of x that an earlier launch of the
+ * same call took on a
  * route without scratch (x runs in pieces of up to 8 rows, and pieces can
  * take different routes) may already have been written, so y is then
  * unspecified (decode shapes need at most a few MiB).  Every call on
@@ -268,7 +270,7 @@ tbh_status tbh_linear_device(const tbh_weight *w, const float *x, int64_t M,
                              int64_t K, const float *bias, float *y, void *stream);
 
 /* Prefill: the same product for M >= 64 rows of bf16 activations, on bf16
- * MFMA (BASELINE configs[3]).  The reference has no bf16 path; it multiplies
+ * MFMA.  The reference has no bf16 path; it multiplies
  * fp32 activations by dequantize(w) with cblas_sgemm
  * (QuantizedTensor.swift:640-642, Tensor.swift:839-861), which is the
  * product computed here for x = the bf16 values widened to fp32: weight
