@@ -2,7 +2,7 @@
 
     python bench.py [--gpus 1] [--steps K] [--warmup W] [--workload NAME]
 
-Default workload (BASELINE.json config 1 at M=1, the config the headline
+Default workload (the one the headline
 metric "dequant-GEMV GB/s and % of HBM peak" is quoted on):
   INT4 weight-only GEMV, symmetric signed 4-bit, one fp32 scale per 32
   consecutive K elements (converter layout), x fp32 [1 x K], for the four
@@ -24,9 +24,9 @@ sgemm on every host CPU this process may use, capped by the CPU share
 OMP_NUM_THREADS grants) on a bounded sample of the same workload.  The
 default line also carries "decode_1p1b_int8": tokens/s of the 1.1B-shaped
 INT8 decode step (the headline metric's second half), same step counts,
-and one key per remaining BASELINE row (TABLE below: INT8 configs[0],
-INT4 configs[1] at M=4 and 8, configs[3] prefill INT8 M=2048 and INT4
-M=512, configs[4] 7B projection set at M=1 and 8 and the 7B decode step),
+and one key per further workload (TABLE below: INT8 decode, INT4 at M=4
+and 8, prefill INT8 M=2048 and INT4 M=512, the 7B projection set at M=1
+and 8 and the 7B decode step),
 each with its own roofline and a bounded CPU baseline sample (a fifth of
 --cpu-budget); --no-table skips them.
 """
@@ -57,7 +57,7 @@ WORKLOADS = {
     "int4_g32_gemv_m1_runtime": ("int4kn", 32, [(2048, 2048), (5632, 2048), (2048, 5632), (32000, 2048)], 1),
 }
 
-# Prefill (BASELINE configs[3]): x [M x K] bf16 N(0,1), one dequant-GEMM on
+# Prefill: x [M x K] bf16 N(0,1), one dequant-GEMM on
 # bf16 MFMA per step.  name: (precision, group, (N, K), M)
 PREFILL = {}
 for _m in (64, 128, 512, 2048):
@@ -68,7 +68,7 @@ for _m in (64, 128, 512, 2048):
 # The same products through the fp32 entry (tbh_matmul_device), the
 # reference's own activation type: x [M x K] fp32 N(0,1).
 PREFILL_F32 = {"prefill_f32_" + k[len("prefill_"):]: v for k, v in PREFILL.items()}
-# Decode (BASELINE configs[2] and [4]): one token of a LLaMA-shaped model on
+# Decode: one token of a LLaMA-shaped model on
 # the GPU decode step.  name: (precision, group, config kwargs, context)
 CFG_7B = dict(num_layers=32, hidden=4096, num_heads=32, num_kv_heads=32, intermediate=11008, vocab=32000)
 DECODE = {
@@ -76,7 +76,7 @@ DECODE = {
                                          intermediate=5632, vocab=32000), 512),
     "decode_7b_int4": ("int4", 32, CFG_7B, 512),
 }
-# The per-token projection set of the 7B shape (BASELINE configs[4], batch
+# The per-token projection set of the 7B shape (batch
 # M in {1, 8}): every layer's q, k, v, o, gate, up and down GEMV and the LM
 # head, each with M rows of x, one step = one token for each of M sequences.
 # name: (precision, group, config kwargs, M)
@@ -100,7 +100,7 @@ OPS = {
 MFMA_BF16_PEAK_TFLOPS = 2500.0  # MI355X dense bf16
 RIDGE_FLOP_PER_BYTE = MFMA_BF16_PEAK_TFLOPS * 1e12 / (HBM_PEAK_GBS * 1e9)
 
-# The rest of the BASELINE table, measured after the headline workload and
+# Further workloads, measured after the headline workload and
 # the 1.1B decode step in the default run, each as a key of the default line
 # with its own roofline and a bounded CPU baseline sample.
 TABLE = ["int8_pc_gemv_m1", "int4_g32_gemv_m4", "int4_g32_gemv_m8", "prefill_int8_m2048", "prefill_int4_m512",
@@ -167,8 +167,7 @@ def pmc_copies(torch, dev):
 
 def host_info() -> dict:
     """Host cores as this process sees them: nproc, the CPUs it may run on,
-    the CPU share the environment grants (OMP_NUM_THREADS; 16 per GPU on the
-    MI355X boxes) and the lscpu model name."""
+    the CPU share the environment grants (OMP_NUM_THREADS) and the lscpu model name."""
     nproc = os.cpu_count() or 1
     try:
         aff = len(os.sched_getaffinity(0))
@@ -982,7 +981,7 @@ def main():
     ap.add_argument("--no-decode", action="store_true",
                     help="int4_g32_gemv_m1: leave out the 1.1B decode-step measurement")
     ap.add_argument("--no-table", action="store_true",
-                    help="int4_g32_gemv_m1: leave out the other BASELINE rows (" + ", ".join(TABLE) + ")")
+                    help="int4_g32_gemv_m1: leave out the further workloads (" + ", ".join(TABLE) + ")")
     ap.add_argument("--trace-summary", metavar="KERNEL_TRACE_CSV",
                     help="summarise a rocprofv3 --kernel-trace CSV (no GPU work): per-kernel averages over "
                          "all dispatches and over the last --last dispatches of kernels matching --kernel")
@@ -1020,11 +1019,11 @@ def main():
     if args.workload == "int4_g32_gemv_m1" and not args.pmc_pass:
         if not args.no_decode:
             # the second half of the headline metric: decode tokens/s at the
-            # 1.1B shape (BASELINE configs[2]), same --steps / --warmup
+            # 1.1B shape, same --steps / --warmup
             _release(torch)
             out["decode_1p1b_int8"] = measure_decode(args, backend, T, torch, "decode_1p1b_int8")
         if not args.no_table:
-            # the rest of the BASELINE table, each row with its roofline and a
+            # the further workloads, each with its roofline and a
             # bounded sample of the reference CPU path
             budget = args.cpu_budget / 5
             for name in TABLE:

@@ -1,5 +1,5 @@
 """bench.py's driver-facing contract, on the CPU (no GPU work): the refusal of
-more than one GPU, the default line's table of BASELINE rows, the counter
+more than one GPU, the default line's table of further workloads, the counter
 records it reads into roofline.traffic, and the kernel-trace summary."""
 import json
 import os
@@ -40,9 +40,9 @@ def test_fp32_prefill_workloads_mirror_the_bf16_ones():
 
 @pytest.mark.parametrize("prec,N,K,M,kind", [
     ("int4", 32000, 2048, 1, ""),            # the headline's dominant launch
-    ("int8", 5632, 2048, 1, ""),             # configs[0]
-    ("int4", 32000, 2048, 8, ""),            # configs[1] at M = 8
-    ("int8", 5632, 2048, 2048, "prefill"),   # configs[3]
+    ("int8", 5632, 2048, 1, ""),             # INT8 decode
+    ("int4", 32000, 2048, 8, ""),            # INT4 decode at M = 8
+    ("int8", 5632, 2048, 2048, "prefill"),   # prefill
     ("int4", 2048, 5632, 512, "prefill"),
 ])
 def test_traffic_records_parse(prec, N, K, M, kind):
@@ -61,7 +61,7 @@ def test_step_traffic_records_parse(workload):
 def test_algorithmic_bytes_closed_forms():
     # INT4 g32: K N / 2 weight bytes + 4 K N / 32 scale bytes + x and y
     assert bench.alg_bytes("int4", 32, 32000, 2048, 1) == 41096192
-    # INT8 per-channel: K N + 4 N + x and y (BASELINE configs[0])
+    # INT8 per-channel: K N + 4 N + x and y
     assert bench.alg_bytes("int8", 0, 5632, 2048, 1) == 11587584
     # prefill: bf16 x
     assert bench.prefill_bytes("int8", 0, 5632, 2048, 512) == 5632 * 2048 + 4 * 5632 + 2 * 512 * 2048 + 4 * 512 * 5632

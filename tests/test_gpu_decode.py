@@ -86,7 +86,7 @@ def test_decode_small(backend, prec):
 
 
 def test_decode_tinyllama_width(backend):
-    # TinyLlama-1.1B layer shapes (BASELINE configs[2]) with 2 of the 22 layers
+    # TinyLlama-1.1B layer shapes with 2 of the 22 layers
     cfg = T.DecoderConfig(num_layers=2, hidden=2048, num_heads=32, num_kv_heads=4, intermediate=5632,
                           vocab=32000, max_seq=64)
     dec, ref = _model(backend, cfg, "int8", seed=21)
@@ -109,7 +109,7 @@ class _Scaled:
 
 
 def test_decode_tinyllama_full_depth(backend):
-    # BASELINE configs[2] at its full depth: 22 layers, hidden 2048, 32/4
+    # TinyLlama-1.1B at its full depth: 22 layers, hidden 2048, 32/4
     # heads, FFN 5632, vocab 32000, INT8 per-channel.  One quantized matrix
     # per projection shape is shared by the layers, with each layer's scales
     # multiplied by 1 + 0.05 l and its own norm weights, so every layer's
@@ -150,7 +150,7 @@ def test_decode_tinyllama_full_depth(backend):
 
 
 def test_decode_tinyllama_context_520(backend):
-    # BASELINE configs[2]'s head layout at its own context: hidden 2048, 32
+    # TinyLlama-1.1B's head layout at context 512: hidden 2048, 32
     # query heads over 4 KV heads (8 per KV head), head_dim 64, FFN 5632,
     # vocab 32000, INT8 per-channel, 2 layers, 520 steps.  Positions 511..519
     # run 16 and 17 attention ranges of 32 positions through the merge, as
@@ -187,7 +187,7 @@ def test_decode_tinyllama_width_runtime_int4(backend):
 
 
 def test_decode_7b_width(backend):
-    # 7B layer shapes (BASELINE configs[4]) with 2 of the 32 layers: INT4
+    # 7B layer shapes with 2 of the 32 layers: INT4
     # group 32 along K, hidden 4096, 32 query and 32 KV heads (head_dim 128,
     # one query head per KV head), FFN 11008, vocab 32000
     cfg = T.DecoderConfig(num_layers=2, hidden=4096, num_heads=32, num_kv_heads=32, intermediate=11008,

@@ -72,7 +72,7 @@ def _int8_pc(seed, K, N, std=0.02):
 
 
 def _int4_nk(seed, K, N, gs, std=0.02):
-    """BASELINE / converter layout: PyTorch [N, K] quantized flat, groups along K."""
+    """Converter layout: PyTorch [N, K] quantized flat, groups along K."""
     w_nk = O.fill_normal(seed, N * K, std=std).reshape(N, K)
     qt = O.quantize_int4(w_nk, gs, O.ROUND_SWIFT)
     qt.shape = (K, N)
@@ -95,7 +95,7 @@ def test_int8_per_channel(backend, K, N):
 
 
 def test_int8_baseline_config0(backend):
-    # BASELINE config 0: W [5632 x 2048] (out x in) -> reference [K=2048, N=5632]
+    # W [5632 x 2048] (out x in) -> reference [K=2048, N=5632]
     qt = _int8_pc(0x7B1A0000, 2048, 5632)
     _check(backend, _product(qt, (2048, 5632)), qt, Ms=(1, 8))
 
@@ -139,7 +139,7 @@ def test_int4_converter_layout(backend, K, N, gs):
 
 @pytest.mark.parametrize("K,N", [(2048, 2048), (2048, 5632), (5632, 2048), (2048, 32000)])
 def test_int4_baseline_config1(backend, K, N):
-    # BASELINE config 1: INT4 g32 along K, shapes [N x K], M in {1, 4, 8}
+    # INT4 g32 along K, shapes [N x K], M in {1, 4, 8}
     qt = _int4_nk(0x7B1A0010 + K + N, K, N, 32)
     _check(backend, _product(qt, (K, N), T.Layout.NK_FLAT), qt, Ms=(1, 4, 8))
 
@@ -202,7 +202,7 @@ def test_burst_k_split(backend, prec, K, N):
     ("int8", 2048, 5632),     # INT8 under 16384 outputs: 8 rows on one burst launch, the GEMM from 9
     ("int8", 2048, 1003),     # ragged N
     ("int8", 1000, 64),       # K off the chunk multiple
-    ("int4", 2048, 2048),     # configs[1] shape the matrix-core GEMV never takes
+    ("int4", 2048, 2048),     # a shape the matrix-core GEMV never takes
     ("int4", 4096, 520),      # two chunk iterations per row: eight staged x rows would need 144 KB
                               # of LDS, so 8 rows run as two 4-row launches (matrix-core GEMV off)
     ("int4kn", 2048, 5632),   # runtime layout (groups along N)
@@ -290,7 +290,7 @@ def test_burst_x_range_extremes(backend, kind, K, N):
 
 @pytest.mark.parametrize("K,N", [(4096, 4096), (4096, 11008), (11008, 4096), (4096, 32000)])
 def test_int4_7b_projection_shapes(backend, K, N):
-    # BASELINE config 4: the 7B projection set (q/k/v/o, gate/up, down, LM
+    # the 7B projection set (q/k/v/o, gate/up, down, LM
     # head), INT4 g32 along K, batch M in {1, 8}; M = 2..4 cross the default
     # VALU / matrix-core thresholds of these shapes
     qt = _int4_nk(0x7B1A0070 + K + N, K, N, 32)
@@ -308,7 +308,7 @@ def test_int4_runtime_layout(backend, K, N, gs, path):
 
 
 @pytest.mark.parametrize("K,N,gs", [
-    (2048, 32000, 32),    # configs[1] shapes in the runtime layout, I = 1, U = 4
+    (2048, 32000, 32),    # decode shapes in the runtime layout, I = 1, U = 4
     (2048, 5632, 32), (5632, 2048, 32),   # I = 3
     (2048, 2048, 64),
     (11008, 4096, 32),    # I = 6 (7B down projection)
@@ -877,7 +877,7 @@ def _prefill_check(backend, pq, oq, M, seed):
 
 
 @pytest.mark.parametrize("prec,K,N,M", [
-    ("int8", 2048, 5632, 64),     # BASELINE configs[3] shapes
+    ("int8", 2048, 5632, 64),     # an FFN projection's shapes
     ("int8", 2048, 5632, 512),
     ("int4", 5632, 2048, 128),
     ("int4", 5632, 2048, 512),
@@ -989,7 +989,7 @@ def test_prefill_bf16_tiles(backend, prec, K, N, M, tile):
 
 
 def test_prefill_bf16_large_m(backend):
-    # configs[3] at M = 2048 (INT4 g32, 2048 x 5632)
+    # a long prompt (INT4 g32, 2048 x 5632)
     oq = _int4_nk(71, 5632, 2048, 32)
     _prefill_check(backend, _product(oq, (5632, 2048), T.Layout.NK_FLAT), oq, 2048, seed=9)
 
@@ -1061,7 +1061,7 @@ def test_prefill_bf16_split_k_determinism_and_graphs(backend):
 
 
 @pytest.mark.parametrize("K,N,gs,M", [
-    (2048, 5632, 32, 512),   # configs[3] shape, Tensor.quantize(.int4): two N-blocks per 64-output tile
+    (2048, 5632, 32, 512),   # Tensor.quantize(.int4): two N-blocks per 64-output tile
     (5632, 2048, 32, 64),    # split along K
     (1000, 384, 128, 129),   # N-blocks of 128 rows (one per tile), K off the 64-deep steps, ragged M
     (512, 320, 64, 300),     # N-blocks of 64 rows

@@ -237,7 +237,7 @@ def quantize_int4_flat(w: np.ndarray, groupSize: int = 32, shape=None,
     """quantizeINT4, QuantizedTensor.swift:502-560, over w's C-order
     flattening (groups of `groupSize` consecutive flat elements).
 
-    For the BASELINE / converter INT4 layout pass the PyTorch [N, K] weight,
+    For the converter's INT4 layout pass the PyTorch [N, K] weight,
     shape=(K, N) and layout=NK_FLAT: groups then run along K."""
     w = np.ascontiguousarray(w, np.float32)
     flat = w.reshape(-1)
