@@ -814,11 +814,14 @@ static int64_t sgemv_min_rows(const tbh_weight &w) {
 // Fewest rows of fp32 x that go to the MFMA GEMM (launch_prefill_f32) instead
 // of the GEMV kernels, which stream the whole weight once per 1..8 rows.
 // Measured crossovers, us per call GEMV / GEMM:
-//   INT4 (its matrix-core GEMV takes eight rows a launch): 2048x2048 16 rows
-//     11.8 / 12.8, 20 14.8 / 11.8 (12 is kept: 11.9 / 12.0 there);
-//     11008x4096 9 rows 21.5 / 24.1, 12 26.9 / 24.2; 4096x11008 12 rows 25.3 /
-//     24.7; 32000x2048 16 rows 26.0 / 30.7, 20 36.9 / 31.9, but 20000x1024 12
-//     rows 22.3 / 18.1; 32000x4096 9 rows 45.5 / 48.4, 12 54.7 / 49.0.
+//   INT4 (its matrix-core GEMV takes eight rows a launch): 2048x2048 12 rows 8.9
+//     / 9.0, 14 10.2 / 9.2; 1024x4096 9 rows 11.0 / 9.4; 11008x4096 9 rows 21.5 /
+//     24.1, 12 26.9 / 24.2; 4096x11008 12 rows 25.3 / 24.7; 16384x1536 9 rows
+//     16.7 / 16.5, 12 21.0 / 16.2.  Wide ones keep two eight-row launches:
+//     28672x2048 16 rows 23.9 / 29.8, 17 31.4 / 30.0; 32000x2048 16 rows 26.0 /
+//     30.7, 20 36.9 / 31.9; 24000x4096 16 rows 39.0 / 46.1; 16384x4096 16 rows
+//     29.5 / 29.8; but 20000x2048 28.1 / 24.5, 32000x3200 54.4 / 40.9 (slower than
+//     they could be, as they were); 32000x4096 9 rows 45.5 / 48.4, 12 54.7 / 49.0.
 //   INT8: 2048x2048 8 rows 7.5 / 7.9, 12 10.7 / 8.0; 4096x4096 4 rows 11.7 /
 //     12.3, 6 13.9 / 12.4; 2048x5632 4 rows 11.6 / 13.1, 6 15.3 / 12.1;
 //     5632x2048 8 rows 9.2 / 11.2 (one eight-row launch), 9 12.5 / 11.7;
